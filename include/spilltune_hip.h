@@ -99,14 +99,18 @@ int st_nf4_dq_scales(const uint8_t* absmax_q, const float* nested_absmax, const 
  *   y[m,n]    = bf16( base + lora_scale * sum_j t[m, seg(n)*rank + j] * lora_b[n,j] )
  *   y[m,n]    = bf16( residual[m,n] + y[m,n] )            (if residual)
  * W [N,K] is payload/scales in flat groups of 128 (64 with ST_FLAG_GROUP64:
- * bitsandbytes' NF4 blocksize, scales from st_nf4_dq_scales), dequantised
- * inside the GEMM and never written to HBM as bf16 (K % group != 0, where
- * the groups straddle W's rows: each packed word reads its own group's
- * scale).  K % 8 == 0.  `workspace`: split-K partials for shapes whose
- * 256x128 tiles leave CUs idle on a long contraction (fp32 [splits, M, N],
- * summed in split order by a second kernel before the epilogue); the query
- * returns the bytes it takes, 0 when the shape runs unsplit.  Without that
- * workspace the call runs unsplit (same epilogue, another fp32 order).
+ * bitsandbytes' NF4 blocksize, scales from st_nf4_dq_scales).  K % 8 == 0.
+ * `workspace`: the query returns the bytes a shape is fastest with, one of
+ *  - 2 N K + 256: many rows; W is decoded to bf16 there once and a bf16 GEMM
+ *    runs on it (the fused kernels decode each W panel once per row tile);
+ *  - split-K partials (fp32 [splits, M, N], summed in split order by a second
+ *    kernel before the epilogue): few outputs, a long contraction;
+ *  - 0: W is dequantised inside the GEMM.
+ * With less the call runs unsplit and dequantises inside the GEMM (K % group
+ * != 0, where the groups straddle W's rows: each packed word reads its own
+ * group's scale).  Decoding first gives the bits of the fused kernels (at
+ * most the last bit of the fp32 LoRA term differs); split-K sums in another
+ * fp32 order.  A workspace belongs to the call until its work on `stream` is done.
  * `t` = x_f32 A_cat^T from st_lora_gemm ([M, nseg*rank] fp32) or NULL for no
  * LoRA; any rank >= 1 (up to 65536 T columns).  The epilogue stages t and
  * lora_b in the tile's LDS; when they do not fit (more than 64 T columns on
@@ -132,8 +136,7 @@ int st_q4_linear_fwd(const uint16_t* x, int64_t M, int64_t K, int64_t ldx,
  * with dt = lora_scale * dy_f32 B ([M, lora_k] fp32, from st_lora_bwd_dy;
  * N-concatenated projections stack their dt columns and lora_a rows) or
  * dt == NULL for no LoRA term; 1 <= lora_k <= 65536 (operands beyond the
- * tile's LDS as in the forward).  W [N,K] as above,
- * dequantised into LDS in its natural orientation and read transposed.
+ * tile's LDS as in the forward).  W [N,K] as above, read transposed.
  * `workspace` as in the forward (the split runs over N).
  */
 int64_t st_q4_linear_dgrad_workspace_bytes(int64_t M, int64_t N, int64_t K);
@@ -151,7 +154,8 @@ int st_q4_linear_dgrad(const uint16_t* dy, int64_t M, int64_t N, int64_t lddy,
  * (the roundings of st_swiglu_bwd) and writes dgu[m, i] = dgate and
  * dgu[m, I + i] = dup (row stride lddgu).  I is this projection's in_features.
  * gu and dgu must be 16-byte aligned with ldgu, lddgu and I multiples of 8
- * (ST_EUNSUPPORTED otherwise).
+ * (ST_EUNSUPPORTED otherwise).  `workspace` as for st_q4_linear_dgrad with
+ * K = I, split-K aside.
  */
 int st_q4_linear_dgrad_swiglu(const uint16_t* dy, int64_t M, int64_t N, int64_t lddy,
                               const uint8_t* payload, const float* scales, int64_t I,

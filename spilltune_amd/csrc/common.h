@@ -27,6 +27,10 @@ void set_error(const char* fmt, ...);
 int fail(int code, const char* fmt, ...);
 int check_launch(const char* what);
 
+// st_dequant4's launch (dequant.hip), arguments checked by the caller
+int launch_dequant4(const uint8_t* payload, const float* scales, int64_t numel, int32_t group,
+                    const float* lut16, int32_t flags, uint16_t* out, hipStream_t stream);
+
 // ---- bf16 helpers ----
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
   return __builtin_bit_cast(float, (uint32_t)h << 16);

@@ -21,12 +21,13 @@
 
 #include "common.h"
 #include "decode4.h"
+#include "gemm_dma.h"
 
 namespace {
 
 constexpr int BK = 64;
 
-enum Mode { FWD_Q4 = 0, DGRAD_Q4 = 1, FWD_BF16 = 2, DGRAD_BF16 = 3 };
+enum Mode { FWD_Q4 = 0, DGRAD_Q4 = 1 };
 
 struct GemmParams {
   const uint16_t* A;
@@ -111,9 +112,7 @@ struct Tile {
   static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
   static constexpr int FM = WM / 32, FN = WN / 32;
   static constexpr int A_IT = BM * 8 / NT;  // 16-byte chunks per thread
-  static constexpr bool Q4 = (MODE == FWD_Q4 || MODE == DGRAD_Q4);
-  static constexpr bool DGRAD = (MODE == DGRAD_Q4 || MODE == DGRAD_BF16);
-  static constexpr int BF_IT = BN * 8 / NT;        // FWD_BF16 chunks per thread
+  static constexpr bool DGRAD = MODE == DGRAD_Q4;
   static constexpr int LDS_CHUNKS = 2 * (BM + BN) * RS;
 };
 
@@ -466,6 +465,232 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, const f32x16 
     blocks(std::false_type{}, std::false_type{});
 }
 
+// Epilogue of the DMA kernels: the same values as gemm_epilogue (bf16(acc),
+// + LoRA, + residual, or the SwiGLU VJP), from 16x16 accumulators (element v
+// of piece (a, b): row 16a + 4*(lane/16) + v, column 16b + lane%16).  A wave
+// works in strips of 32 rows x all its columns, so each staged T value feeds
+// every column piece, and stages 32x32 blocks for 16-byte rows as there.
+// The fp32 LoRA product (v_mfma_f32_16x16x4_f32, 1/16 of the bf16 rate) alone
+// takes 4 us per 256x256 tile at rank 16.
+template <bool DGRAD, int BM, int BN, int NT, int FM, int FN>
+__device__ __forceinline__ void dma_epilogue(const GemmParams& p, const f32x4 (&acc)[FM][FN],
+                                             uint4* lds, int m0, int mend, int p0, int wr, int wc,
+                                             int tid, int lane) {
+  const bool lora = p.T != nullptr;
+  float* Ts = (float*)lds;
+  const int tstride = p.lora_cols + 1;
+  float* Ls = Ts + BM * tstride;
+  const int lstride = DGRAD ? BN : (p.lora_k + 1);
+  const int P = (int)p.P;
+  if (lora) {
+    stage_f32<NT>(Ts, tstride, make_rsrc(p.T, 0x7fffffff), p.ldt, m0, 0, BM, p.lora_cols,
+                  mend - m0, p.lora_cols, tid);
+    if (DGRAD)
+      stage_f32<NT>(Ls, lstride, make_rsrc(p.L, 0x7fffffff), p.ldl, 0, p0, p.lora_k, BN, p.lora_k,
+                    P - p0, tid);
+    else
+      stage_f32<NT>(Ls, lstride, make_rsrc(p.L, 0x7fffffff), p.ldl, p0, 0, BN, p.lora_k, P - p0,
+                    p.lora_k, tid);
+    __syncthreads();
+  }
+  const auto rsC = make_rsrc(p.C, 0x7fffffff);
+  const auto rsR = make_rsrc(p.R, 0x7fffffff);
+  const auto rsG = make_rsrc(p.swi_gu, 0x7fffffff);
+  const uint32_t ldc2 = (uint32_t)p.ldc * 2, ldr2 = (uint32_t)p.ldr * 2;
+  uint32_t* stg = (uint32_t*)lds + epi_stage_offset<DGRAD, BM, BN>(p) + (tid >> 6) * EPI_STG;
+  const int l = lane & 15, g = lane >> 4;
+  const int q = l, kc = g;  // vector form: this lane's row pair and 8-column group of a block
+
+  // T column offset of the segment that 32-column block j belongs to
+  auto seg_off = [&](int cl) {
+    int coff = 0;
+    if (!DGRAD)
+      for (int i = 0; i < p.nseg; ++i) coff += p.seg_end[i] <= p0 + cl ? p.lora_k : 0;
+    return coff;
+  };
+  // fp32 LoRA product of a 32-row strip, the rank four at a time; ranks past
+  // the last are selected to zero (other values are staged there)
+  f32x4 la[2][FN];
+  auto lora_strip = [&](int rl) {
+    int coff[FN / 2];
+#pragma unroll
+    for (int j = 0; j < FN / 2; ++j) coff[j] = seg_off(wc + 32 * j);
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < FN; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) la[a][b][v] = 0.0f;
+    for (int kk = 0; kk < p.lora_k; kk += 4) {
+      const bool in = kk + g < p.lora_k;
+      const int kx = in ? kk + g : 0;
+      float av[2][FN / 2], bv[FN];
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int j = 0; j < FN / 2; ++j) {
+          const float t = Ts[(rl + 16 * a + l) * tstride + coff[j] + kx];
+          av[a][j] = in ? t : 0.0f;
+        }
+#pragma unroll
+      for (int b = 0; b < FN; ++b) {
+        const int col = wc + 16 * b + l;
+        const float r = DGRAD ? Ls[kx * lstride + col] : Ls[col * lstride + kx];
+        bv[b] = in ? r : 0.0f;
+      }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < FN; ++b)
+          la[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a][b / 2], bv[b], la[a][b], 0, 0, 0);
+    }
+  };
+  auto finish = [&](float av, float lv) {
+    float y = st::bf16r(av);
+    if (lora) {
+      if (DGRAD)
+        y = st::bf16r(y + st::bf16r(lv));
+      else
+        y = st::bf16r(y + lv * p.lora_scale);
+    }
+    return y;
+  };
+  // operands of 32x32 block (i, j) for this lane's rows 2q, 2q+1: residual
+  // rows in a0, a1, or (SWI) gate rows in a0, a1 and up rows in b0, b1
+  auto fetch = [&](auto swi, int i, int j) {
+    const int row0 = m0 + wr + i * 32 + 2 * q, col = p0 + wc + j * 32 + 8 * kc;
+    const bool cok = col < P, ok0 = cok && row0 < mend, ok1 = cok && row0 + 1 < mend;
+    EpiIn in;
+    in.a0 = in.a1 = in.b0 = in.b1 = make_uint4(0, 0, 0, 0);
+    if constexpr (decltype(swi)::value) {
+      const uint32_t ldg2 = (uint32_t)p.swi_ld * 2, uo = (uint32_t)p.swi_I * 2;
+      const uint32_t gb = (uint32_t)row0 * ldg2 + (uint32_t)col * 2;
+      in.a0 = ld16(rsG, ok0 ? gb : kOOB);
+      in.a1 = ld16(rsG, ok1 ? gb + ldg2 : kOOB);
+      in.b0 = ld16(rsG, ok0 ? gb + uo : kOOB);
+      in.b1 = ld16(rsG, ok1 ? gb + ldg2 + uo : kOOB);
+    } else if (p.R) {
+      const uint32_t rb = (uint32_t)row0 * ldr2 + (uint32_t)col * 2;
+      in.a0 = ld16(rsR, ok0 ? rb : kOOB);
+      in.a1 = ld16(rsR, ok1 ? rb + ldr2 : kOOB);
+    }
+    return in;
+  };
+  auto store16 = [&](const uint32_t (&o)[4], bool ok, uint32_t off) {
+    __builtin_amdgcn_raw_buffer_store_b128(st::u32x4{o[0], o[1], o[2], o[3]}, rsC,
+                                           (int)(ok ? off : kOOB), 0, 0);
+  };
+  auto vec_blocks = [&](auto swi) {
+    constexpr bool SWI = decltype(swi)::value;
+    constexpr int BJ = FN / 2;
+    EpiIn cur = fetch(swi, 0, 0);
+#pragma unroll
+    for (int i = 0; i < FM / 2; ++i) {
+      if (lora) lora_strip(wr + 32 * i);
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) {
+        const int row0 = m0 + wr + i * 32 + 2 * q, col = p0 + wc + j * 32 + 8 * kc;
+        const bool cok = col < P, ok0 = cok && row0 < mend, ok1 = cok && row0 + 1 < mend;
+        // this block's operands were issued one block ahead; issue the next one's
+        const EpiIn in = cur;
+        if (i * BJ + j + 1 < FM / 2 * BJ) cur = fetch(swi, (i * BJ + j + 1) / BJ, (j + 1) % BJ);
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+              const f32x4 &c = acc[2 * i + a][2 * j + b], &r = la[a][2 * j + b];
+              const int pr = 8 * a + 2 * g + t;  // row pair
+              stg[pr * 36 + 16 * b + l] = st::pack_bf16x2(finish(c[2 * t], r[2 * t]),
+                                                          finish(c[2 * t + 1], r[2 * t + 1]));
+            }
+        // the wave reads back only its own area: LDS accesses of one wave
+        // complete in order, the fence keeps the compiler from moving them
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        const uint4 lo4 = *(const uint4*)&stg[q * 36 + 8 * kc];
+        const uint4 hi4 = *(const uint4*)&stg[q * 36 + 8 * kc + 4];
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // before the next block's writes
+        // dword c of the pair holds (row 2q, row 2q+1) of column 8kc + c
+        const uint32_t d[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+        const uint32_t cb = (uint32_t)row0 * ldc2 + (uint32_t)col * 2;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const bool ok = r ? ok1 : ok0;
+          const uint32_t off = r ? cb + ldc2 : cb;
+          uint32_t e[4];
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            e[c] = __builtin_amdgcn_perm(d[2 * c + 1], d[2 * c], r ? 0x07060302u : 0x05040100u);
+          const uint4 &x = r ? in.a1 : in.a0, &u = r ? in.b1 : in.b0;
+          const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, uw[4] = {u.x, u.y, u.z, u.w};
+          if constexpr (SWI) {
+            // SwiGLU VJP of dense.py:153 on the bf16 dX value (st::swiglu_vjp,
+            // as the standalone SwiGLU backward)
+            uint32_t og[4], ou[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              float rg[2], ru[2];
+#pragma unroll
+              for (int h = 0; h < 2; ++h)
+                st::swiglu_vjp(st::bf16_to_f32((uint16_t)(xw[c] >> (16 * h))),
+                               st::bf16_to_f32((uint16_t)(uw[c] >> (16 * h))),
+                               st::bf16_to_f32((uint16_t)(e[c] >> (16 * h))), rg[h], ru[h]);
+              og[c] = st::pack_bf16x2(rg[0], rg[1]);
+              ou[c] = st::pack_bf16x2(ru[0], ru[1]);
+            }
+            store16(og, ok, off);
+            store16(ou, ok, off + (uint32_t)p.swi_I * 2);
+          } else {
+            if (p.R) {
+#pragma unroll
+              for (int c = 0; c < 4; ++c)
+                e[c] = st::pack_bf16x2(
+                    st::bf16_to_f32((uint16_t)xw[c]) + st::bf16_to_f32((uint16_t)e[c]),
+                    st::bf16_to_f32((uint16_t)(xw[c] >> 16)) +
+                        st::bf16_to_f32((uint16_t)(e[c] >> 16)));
+            }
+            store16(e, ok, off);
+          }
+        }
+      }
+    }
+  };
+  if constexpr (DGRAD) {
+    if (p.swi_gu) {  // the launcher only sets swi_gu with vec_epi
+      vec_blocks(std::true_type{});
+      return;
+    }
+  }
+  if (p.vec_epi) {
+    vec_blocks(std::false_type{});
+    return;
+  }
+  // one 2-byte access per element
+#pragma unroll
+  for (int i = 0; i < FM / 2; ++i) {
+    if (lora) lora_strip(wr + 32 * i);
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < FN; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = m0 + wr + 32 * i + 16 * a + 4 * g + v, col = p0 + wc + 16 * b + l;
+          const bool ok = row < mend && col < P;
+          float y = finish(acc[2 * i + a][b][v], la[a][b][v]);
+          if (p.R)
+            y = st::bf16r(st::bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(
+                              rsR, (int)(ok ? (uint32_t)row * ldr2 + (uint32_t)col * 2 : kOOB), 0,
+                              0)) +
+                          y);
+          __builtin_amdgcn_raw_buffer_store_b16(
+              st::f32_to_bf16(y), rsC, (int)(ok ? (uint32_t)row * ldc2 + (uint32_t)col * 2 : kOOB),
+              0, 0);
+        }
+  }
+}
+
 // FLAT (4-bit modes, 128x128 tiles): K is not a multiple of the scale group
 // (128, or 64 with gshift 6), so the flat groups of W straddle its rows; every
 // packed word (8 weights, which K % 8 == 0 keeps inside one group) then reads
@@ -501,8 +726,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_kernel(GemmParams p) {
   // ---- buffer resources: out-of-range loads return zero, so the main loop
   // needs no bounds branches (rows beyond M/P and the contraction tail).
   const auto rsA = make_rsrc(p.A, p.a_bytes);
-  const auto rsW = make_rsrc(TL::Q4 ? (const void*)(p.Wq + grp * p.w_gstride)
-                                     : (const void*)(p.Wb + grp * p.w_gstride), p.w_bytes);
+  const auto rsW = make_rsrc(p.Wq + grp * p.w_gstride, p.w_bytes);
   const auto rsS = make_rsrc(p.Ws + grp * p.s_gstride, p.s_bytes);
   const float* Lg = p.L + grp * p.l_gstride;
 
@@ -551,16 +775,14 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_kernel(GemmParams p) {
   // B operand source.  FWD_Q4: thread owns EPT consecutive weights of one W row.
   constexpr int TPR = NT / BN;          // threads per W row (1, 2 or 4)
   constexpr int EPT = BK / TPR;         // elements per thread per k-step (64, 32 or 16)
-  // DGRAD_Q4 / DGRAD_BF16: the B tile is W[n][k] for BK contraction rows n
-  // and BN output columns k, kept in that (natural) orientation; each thread
-  // dequantises (or copies) DE consecutive k of one row n, and the MFMA
-  // operand is read transposed.
+  // DGRAD_Q4: the B tile is W[n][k] for BK contraction rows n and BN output
+  // columns k, kept in that (natural) orientation; each thread dequantises
+  // DE consecutive k of one row n, and the MFMA operand is read transposed.
   constexpr int DE = BN * BK / NT;      // dgrad elements per thread per k-step (32 or 16)
   constexpr int DTR = BN / DE;          // dgrad threads per contraction row
   // packed 4-bit words (8 codes each) per thread per k-step
-  constexpr int NW = MODE == FWD_Q4 ? EPT / 8 : MODE == DGRAD_Q4 ? DE / 8 : 1;
-  static_assert(!TL::Q4 || NW == 2 || NW % 4 == 0, "packed W loads are 8 bytes or whole 16-byte pieces");
-  constexpr int WQ = TL::Q4 ? 1 : (TL::DGRAD ? DE / 8 : TL::BF_IT);
+  constexpr int NW = (MODE == FWD_Q4 ? EPT : DE) / 8;
+  static_assert(NW == 2 || NW % 4 == 0, "packed W loads are 8 bytes or whole 16-byte pieces");
   const int brow = tid / TPR, bsub = tid % TPR;       // FWD_Q4 mapping
   const int drow = tid / DTR, dsub = tid % DTR;       // dgrad mapping
   // FWD_Q4 byte offsets at k = 0 of the thread's packed weights and of its
@@ -581,16 +803,14 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_kernel(GemmParams p) {
   const bool dcol_ok = p0 + dsub * DE < p.P;
   static_assert(!TL::DGRAD || NT / DTR == BK, "dgrad: one thread row per contraction row");
 
-  static_assert(!FLAT || (TL::Q4 && BM == 128 && BN == 128), "FLAT: 4-bit 128x128 tiles only");
+  static_assert(!FLAT || (BM == 128 && BN == 128), "FLAT: 4-bit 128x128 tiles only");
   // DGRAD_Q4 with 128-wide B rows: each thread's 4 words are dequantised and
   // stored in an order rotated by its group dsub, free of LDS bank conflicts
   // with st::trswz<128> (every store instruction of a quarter-wave then
   // writes each 4-chunk group's chunk (ch + group) & 3)
   constexpr bool DROT = MODE == DGRAD_Q4 && BN == 128 && NW == 4 && DTR == 4;
-  static_assert(MODE != DGRAD_BF16 || WQ * (NT / (BN / 8)) == BK, "DGRAD_BF16: whole rows per thread block");
   struct WRegs {
-    uint4 q[WQ];      // bf16 modes
-    uint32_t w[NW];   // 4-bit modes
+    uint32_t w[NW];
     float s[FLAT ? NW : 1];  // scale of the tile's group, or of each word (FLAT)
   };
   // NW packed words from byte offset po (kOOB: zeros)
@@ -621,15 +841,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_kernel(GemmParams p) {
       } else {
         w.s[0] = __builtin_bit_cast(float, ld4(rsS, w_so + (uint32_t)(kt >> gstep) * 4));
       }
-    } else if constexpr (MODE == FWD_BF16) {
-#pragma unroll
-      for (int i = 0; i < WQ; ++i) {
-        int id = tid + i * NT, row = id >> 3, c = id & 7;
-        int64_t n = p0 + row;
-        int k = kt * BK + c * 8;
-        w.q[i] = ld16(rsW, (n < p.P && k < p.Q) ? (uint32_t)((n * p.ldw + k) * 2) : kOOB);
-      }
-    } else if constexpr (MODE == DGRAD_Q4) {
+    } else {
       const int64_t n = (int64_t)kt * BK + drow;
       const bool ok = dcol_ok && n < p.Q;
       // DE-aligned: one scale group unless FLAT
@@ -642,16 +854,6 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_kernel(GemmParams p) {
         st::rot4(w.w, dsub);
         if constexpr (FLAT) st::rot4(w.s, dsub);
       }
-    } else {  // DGRAD_BF16: chunk (row, tid % CPR) for rows tid / CPR + i * NT / CPR
-      // (whole 16-byte-chunk rows per load instruction)
-      constexpr int CPR = BN / 8;
-      const int64_t col = p0 + (tid % CPR) * 8;
-#pragma unroll
-      for (int i = 0; i < WQ; ++i) {
-        const int64_t n = (int64_t)kt * BK + tid / CPR + i * (NT / CPR);
-        const bool ok = n < p.Q && col < p.P;
-        w.q[i] = ld16(rsW, ok ? (uint32_t)((n * p.ldw + col) * 2) : kOOB);
-      }
     }
   };
 
@@ -659,40 +861,26 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_kernel(GemmParams p) {
   Tbl tbl;
   const uint32_t sh_e = p.hi_first ? 4u : 0u;
   auto store_B_part = [&](uint4* bs, const WRegs& w, int part) {
-    if constexpr (TL::Q4) {
-      // 8-element chunk ch goes out in quarter ch*4/NW (two chunks per quarter
-      // for NW = 8, quarters 0 and 2 for NW = 2)
+    // 8-element chunk ch goes out in quarter ch*4/NW (two chunks per quarter
+    // for NW = 8, quarters 0 and 2 for NW = 2)
 #pragma unroll
-      for (int ch = 0; ch < NW; ++ch) {
-        if (ch * 4 / NW != part) continue;
-        uint32_t o[4];
-        if constexpr (FLAT)
-          deq8(w.w[ch], make_tbl(p.lut, w.s[ch]), sh_e, 4u - sh_e, o);
-        else
-          deq8(w.w[ch], tbl, sh_e, 4u - sh_e, o);
-        const int ot = fresh_tid();
-        const int idx =
-            MODE == FWD_Q4 ? pad(ot / TPR, ((ot % TPR) * EPT) / 8 + ch)
-            : DROT         ? dswz(ot / DTR, (ot % DTR) * NW + ((ch + ot % DTR) & 3))
-                           : dswz(ot / DTR, (ot % DTR) * NW + ch);
-        bs[idx] = make_uint4(o[0], o[1], o[2], o[3]);
-      }
-    } else if constexpr (MODE == FWD_BF16) {
-#pragma unroll
-      for (int i = 0; i < WQ; ++i) {
-        if (i * 4 / WQ != part) continue;
-        int id = tid + i * NT;
-        bs[pad(id >> 3, id & 7)] = w.q[i];
-      }
-    } else {  // DGRAD_BF16: the loaded chunks as they lie, transposed-operand layout
-      constexpr int CPR = BN / 8;
+    for (int ch = 0; ch < NW; ++ch) {
+      if (ch * 4 / NW != part) continue;
+      uint32_t o[4];
+      if constexpr (FLAT)
+        deq8(w.w[ch], make_tbl(p.lut, w.s[ch]), sh_e, 4u - sh_e, o);
+      else
+        deq8(w.w[ch], tbl, sh_e, 4u - sh_e, o);
       const int ot = fresh_tid();
-      if (part < WQ)
-        bs[dswz(ot / CPR + part * (NT / CPR), ot % CPR)] = w.q[part < WQ ? part : 0];
+      const int idx =
+          MODE == FWD_Q4 ? pad(ot / TPR, ((ot % TPR) * EPT) / 8 + ch)
+          : DROT         ? dswz(ot / DTR, (ot % DTR) * NW + ((ch + ot % DTR) & 3))
+                         : dswz(ot / DTR, (ot % DTR) * NW + ch);
+      bs[idx] = make_uint4(o[0], o[1], o[2], o[3]);
     }
   };
   auto prep_B = [&](const WRegs& w) {
-    if constexpr (!FLAT && (MODE == FWD_Q4 || MODE == DGRAD_Q4)) tbl = make_tbl(p.lut, w.s[0]);
+    if constexpr (!FLAT) tbl = make_tbl(p.lut, w.s[0]);
   };
 
   f32x16 acc[FM][FN];
@@ -794,19 +982,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_kernel(GemmParams p) {
                                                        lane, true, Lg);
 }
 
-// s_waitcnt for at most VM vector-memory and LGKM LDS/scalar operations in
-// flight (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt 7 = no wait,
-// lgkmcnt in bits 11:8; VM = 63 / LGKM = 15 leave that counter alone)
-template <int VM, int LGKM = 15>
-__device__ __forceinline__ void wait_cnt() {
-  static_assert(VM >= 0 && VM < 64 && LGKM >= 0 && LGKM < 16, "counter range");
-  __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | (LGKM << 8) | ((VM >> 4) << 14));
-}
-// Workgroup barrier without the fence of __syncthreads (which would also wait
-// for every LDS DMA in flight): the caller first waits for exactly the
-// operations other waves depend on.  The memory clobber keeps the compiler
-// from moving memory accesses across it.
-__device__ __forceinline__ void bar() { asm volatile("s_barrier" ::: "memory"); }
+using st::bar;
+using st::wait_cnt;
 
 // Warp-specialised 256x128 tile, 8 waves in two roles.  Waves 0-3 (one per
 // SIMD) only read operand fragments and issue MFMAs on a 2x2 grid of 128x64
@@ -1355,6 +1532,30 @@ __global__ __launch_bounds__(64 * WAVES, FM == 4 ? 4 : 1) void gemm_rb_kernel(Ge
                                                    true, p.L + grp * p.l_gstride);
 }
 
+// bf16 x bf16 GEMM with both operands moved by DMA (gemm_dma.h): the plain
+// bf16 linears, and the 4-bit linears whose W was decoded into a workspace.
+template <class LP>
+__global__ __launch_bounds__(LP::NT, LP::MIN_WG_WAVES) void gemm_dma_kernel(GemmParams p) {
+  constexpr bool NN = LP::NN_B;
+  __shared__ uint4 lds[LP::LDS16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int M = (int)p.M, P = (int)p.P;
+  // st::xcd_remap and st::raster in 32 bits (64-bit divisions cost ~1 us here)
+  const unsigned nb = gridDim.x, tiles_m = (M + LP::BM - 1) / LP::BM,
+                 tiles_p = (P + LP::BN - 1) / LP::BN;
+  unsigned t = blockIdx.x;
+  if (nb % 8 == 0) t = (t % 8) * (nb / 8) + t / 8;
+  const unsigned per = (unsigned)p.raster_m * tiles_p, r0 = t / per * p.raster_m, r = t % per;
+  const unsigned h = min(tiles_m - r0, (unsigned)p.raster_m);
+  const int m0 = (int)(r0 + r % h) * LP::BM, p0 = (int)(r / h) * LP::BN;
+  const st::DmaOperands o{p.A, p.Wb, p.lda, p.ldw, p.a_bytes, p.w_bytes};
+  f32x4 acc[LP::FM][LP::FN];
+  LP::run(o, lds, m0, M, p0, P, (int)p.Q, wave, lane, acc);
+  dma_epilogue<NN, LP::BM, LP::BN, LP::NT, LP::FM, LP::FN>(
+      p, acc, lds, m0, M, p0, wave / LP::WAVES_N * LP::WM, wave % LP::WAVES_N * LP::WN, tid, lane);
+}
+
 // Chooses the epilogue's access width (GemmParams::vec_epi): 16-byte rows
 // need C, the residual and gate|up 16-byte aligned with row strides, P and
 // the gate|up split multiples of 8, and `waves` staging areas after the LoRA
@@ -1471,7 +1672,7 @@ int launch(const GemmParams& p, hipStream_t stream) {
   // memory runs the GEMM
   if constexpr (LG) {
     q.lora_global = q.T ? 1 : 0;
-  } else if constexpr (TL::Q4) {
+  } else {
     if (!lora_staged_fits<TL::DGRAD, BM, BN>(q, (int64_t)TL::LDS_CHUNKS * 4, WAVES))
       return launch<MODE, 128, 128, 4, 2, FLAT, true>(p, stream);
   }
@@ -1635,64 +1836,203 @@ int launch_ws_split(GemmParams p, const SplitPlan& plan, void* workspace, hipStr
   return st::check_launch("q4gemm split-K epilogue");
 }
 
+bool al16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
+
+// Whether a fused forward takes the register-operand 256x256 tile: unless
+// ST_GEMM_RB=0, where its whole ring of k-steps and 128-element groups fit.
+bool rb_fits(const GemmParams& p) {
+  const char* rbe = getenv("ST_GEMM_RB");
+  return (!rbe || atoi(rbe)) && p.Q % (RB_ST * BK) == 0 && p.gshift == 7;
+}
+bool forward_runs_rb(const GemmParams& p) {
+  constexpr int64_t lds_dwords = (int64_t)RB_ST * 256 * BK / 8 * 4;
+  return tile_choice(FWD_Q4, p.M, p.P) == 256 && rb_fits(p) && al16(p.Wq) &&
+         lora_staged_fits<false, 256, 256>(p, lds_dwords, 8);
+}
+
 template <int MODE>
 int dispatch(const GemmParams& p, hipStream_t stream) {
-  // the dense-W fallbacks (K not a multiple of 128) always use 128x128 tiles
-  if constexpr (MODE == FWD_Q4 || MODE == DGRAD_Q4) {
-    const int t = tile_choice(MODE, p.M, p.P);
-    if constexpr (MODE == FWD_Q4) {
-      // 256x256 forward: register-operand kernel (8 waves) unless
-      // ST_GEMM_RB=0; its column tail runs on the register-operand 256x128
-      // tile, which sums each output in the same order, so a split stays
-      // bit-identical to one launch
-      const char* rbe = getenv("ST_GEMM_RB");
-      const bool rb = (!rbe || atoi(rbe)) && p.Q % (RB_ST * BK) == 0 && p.gshift == 7;
-      if (const int64_t c1 = split_column(t, p.M, p.P)) {
-        const GemmParams head = column_slice(p, 0, c1), tail = column_slice(p, c1, p.P);
-        if (rb) {
-          const int rc = launch_rb<1, 8>(head, stream);
-          return rc ? rc : launch_rb<1, 4>(tail, stream);
-        }
-        const int rc = launch<MODE, 256, 256, 8>(head, stream);
-        return rc ? rc : launch_ws<MODE>(tail, stream);
+  const int t = tile_choice(MODE, p.M, p.P);
+  if constexpr (MODE == FWD_Q4) {
+    // 256x256 forward: register-operand kernel (8 waves) unless
+    // ST_GEMM_RB=0; its column tail runs on the register-operand 256x128
+    // tile, which sums each output in the same order, so a split stays
+    // bit-identical to one launch
+    const bool rb = rb_fits(p);
+    if (const int64_t c1 = split_column(t, p.M, p.P)) {
+      const GemmParams head = column_slice(p, 0, c1), tail = column_slice(p, c1, p.P);
+      if (rb) {
+        const int rc = launch_rb<1, 8>(head, stream);
+        return rc ? rc : launch_rb<1, 4>(tail, stream);
       }
-      if (t == 256 && rb) return launch_rb<1, 8>(p, stream);
+      const int rc = launch<MODE, 256, 256, 8>(head, stream);
+      return rc ? rc : launch_ws<MODE>(tail, stream);
     }
-    if (t == 256) return launch<MODE, 256, 256, 8>(p, stream);
-    if (t == 2562) return launch_ws<MODE>(p, stream);
-    if constexpr (MODE == FWD_Q4) {
-      const bool rbk = p.Q % (RB_ST * BK) == 0 && p.gshift == 7;
-      if (t == 2566 && rbk) return launch_rb<1, 8>(p, stream);
-      if (t == 2567 && rbk) return launch_rb<1, 4>(p, stream);
-      if (t == 2568 && rbk) return launch_rb<1, 8, 4>(p, stream);
-    }
+    if (t == 256 && rb) return launch_rb<1, 8>(p, stream);
+  }
+  if (t == 256) return launch<MODE, 256, 256, 8>(p, stream);
+  if (t == 2562) return launch_ws<MODE>(p, stream);
+  if constexpr (MODE == FWD_Q4) {
+    const bool rbk = p.Q % (RB_ST * BK) == 0 && p.gshift == 7;
+    if (t == 2566 && rbk) return launch_rb<1, 8>(p, stream);
+    if (t == 2567 && rbk) return launch_rb<1, 4>(p, stream);
+    if (t == 2568 && rbk) return launch_rb<1, 8, 4>(p, stream);
   }
   return launch<MODE, 128, 128, 4>(p, stream);
 }
 
-int run_gemm(int mode, const GemmParams& p, hipStream_t stream) {
-  switch (mode) {
-    case FWD_Q4: return dispatch<FWD_Q4>(p, stream);
-    case DGRAD_Q4: return dispatch<DGRAD_Q4>(p, stream);
-    case FWD_BF16: return dispatch<FWD_BF16>(p, stream);
-    default: return dispatch<DGRAD_BF16>(p, stream);
+// ---- bf16 GEMM on the DMA tiles
+enum DmaKind { DMA_256 = 256, DMA_256x128 = 2561, DMA_128 = 128 };
+
+template <class LP>
+int launch_dma_tile(GemmParams p, hipStream_t stream) {
+  const int64_t tiles = st::cdiv(p.M, LP::BM) * st::cdiv(p.P, LP::BN);
+  if (tiles > 0x7fffffff) return st::fail(ST_EUNSUPPORTED, "q4gemm: too many tiles");
+  if (int rc = check_epilogue_extents(p)) return rc;
+  p.raster_m = raster_choice(p);
+  if (int rc = choose_epilogue<LP::NN_B, LP::BM, LP::BN>(p, (int64_t)LP::LDS16 * 4, LP::WAVES)) return rc;
+  gemm_dma_kernel<LP><<<(unsigned)tiles, LP::NT, 0, stream>>>(p);
+  return st::check_launch("gemm_dma");
+}
+
+// Modelled microseconds of `n` tiles on `slots` at once: whole rounds of `hi`
+// per 64-deep k-step, a last round between `lo` and `hi` with its fill.
+double rounds_us(int64_t n, int64_t slots, double lo, double hi, double ks) {
+  const int64_t rest = n % slots;
+  const double occ = (double)rest / (double)slots;
+  return (double)(n / slots) * (hi * ks + 5) +
+         (rest ? (lo + (hi - lo) * occ * occ * occ) * ks + 5 : 0);
+}
+
+// Tile of a DMA GEMM: the one with the least modelled time.  Microseconds per
+// k-step and round, measured over M = 256..4096 at the four projection shapes
+// of a 4096/14336-wide layer (transposed B in brackets): a 256x256 tile 1.12
+// (1.15) on a half-idle chip rising to 1.45 (1.5) with every CU busy, where
+// the clock drops (2048 x 4096 x 4096 79 us, 4096 x 4096 x 4096 98); 256x128
+// 0.68 to 0.83 (0.72 to 0.88; 2048 x 4096 x 4096 58 us); a pair of 128x128
+// tiles on a CU 0.7 to 0.87, one alone 0.63 (512 x 4096 x 4096 47 us).
+// ST_GEMM_DMA = 256, 2561 or 128 pins a tile for the tests.
+DmaKind dma_kind(bool nn, int64_t M, int64_t P, int64_t Q, double* us = nullptr) {
+  const double ks = (double)st::cdiv(Q, BK);
+  const int64_t cus = cu_count(), n128 = st::cdiv(M, 128) * st::cdiv(P, 128);
+  const double c256 = rounds_us(st::cdiv(M, 256) * st::cdiv(P, 256), cus, nn ? 1.15 : 1.12,
+                                nn ? 1.5 : 1.45, ks);
+  const double c2561 = rounds_us(st::cdiv(M, 256) * st::cdiv(P, 128), cus, nn ? 0.72 : 0.68,
+                                 nn ? 0.88 : 0.83, ks);
+  const double c128 = n128 <= cus ? (nn ? 0.68 : 0.63) * ks + 5
+                                  : rounds_us(n128, 2 * cus, nn ? 0.72 : 0.7, nn ? 0.92 : 0.87, ks);
+  DmaKind k = DMA_256;
+  double c = c256;
+  if (c2561 < c) c = c2561, k = DMA_256x128;
+  if (c128 < c) c = c128, k = DMA_128;
+  if (us) *us = c;
+  const char* env = getenv("ST_GEMM_DMA");
+  const int e = env ? atoi(env) : 0;
+  return e == DMA_256 || e == DMA_256x128 || e == DMA_128 ? (DmaKind)e : k;
+}
+
+// PERM: the contraction order of the register-operand forward (gemm_dma.h)
+template <bool NN, bool PERM = false>
+int launch_dma(const GemmParams& p, hipStream_t stream) {
+  switch (dma_kind(NN, p.M, p.P, p.Q)) {
+    case DMA_256: return launch_dma_tile<st::DmaLoop256<NN, PERM>>(p, stream);
+    case DMA_256x128: return launch_dma_tile<st::DmaLoop64<NN, PERM, 4, 2, 3>>(p, stream);
+    default: return launch_dma_tile<st::DmaLoop64<NN, PERM, 2, 2, 2>>(p, stream);
   }
 }
 
-bool al16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
+// Whether the LoRA operands (and the SwiGLU staging) fit the chosen tile.
+template <bool NN>
+bool dma_lora_fits(const GemmParams& p) {
+  switch (dma_kind(NN, p.M, p.P, p.Q)) {
+    case DMA_256:
+      return lora_staged_fits<NN, 256, 256>(p, (int64_t)st::DmaLoop256<NN, false>::LDS16 * 4, 8);
+    case DMA_256x128:
+      return lora_staged_fits<NN, 256, 128>(p, (int64_t)st::DmaLoop64<NN, false, 4, 2, 3>::LDS16 * 4, 8);
+    default:
+      return lora_staged_fits<NN, 128, 128>(p, (int64_t)st::DmaLoop64<NN, false, 2, 2, 2>::LDS16 * 4, 4);
+  }
+}
+
+// Whether a dense 4-bit linear decodes W into the workspace once and runs the
+// DMA GEMM on it (the fused kernels decode every W panel once per row tile).
+// Both sides are modelled from the same measurements: the decode moves 2.53 B
+// a weight at 4.7 TB/s; the fused kernels take, per k-step and round, 1.4 to
+// 1.72 us for a 256x256 forward tile, 0.85 to 1.04 for the warp-specialised
+// 256x128 and 0.85 (dgrad 0.8) for 128x128, half as much again where scale
+// groups straddle W's rows.  At 2048 rows of a 4096/14336-wide layer with
+// rank-16 LoRA, fused against decode + GEMM: down forward 252 -> 223 us, o 85
+// -> 75, down dgrad with the SwiGLU VJP 319 -> 272, gate|up forward 478
+// against 472; at 2103 rows (a ninth row tile) down 407 -> 275, gate|up dgrad
+// 789 -> 564; at 4096 rows gate|up forward 802 -> 753, dgrad 929 -> 719.  Few
+// rows of a wide W stay fused (256 rows of gate|up 76 against 128), as do
+// fewer than 256 rows and split-K shapes (few outputs, long contraction).
+// ST_GEMM_DECODE = 0 or 1 overrides the model.
+template <int MODE>
+bool decode_first(int64_t M, int64_t P, int64_t Q) {
+  if (getenv("ST_GEMM_TILE")) return false;
+  const char* env = getenv("ST_GEMM_DECODE");
+  if (env) return atoi(env) != 0;
+  if (M < 256 || split_plan(M, P, Q).splits > 1) return false;
+  constexpr bool NN = MODE == DGRAD_Q4;
+  double dma;
+  dma_kind(NN, M, P, Q, &dma);
+  dma += (double)P * (double)Q * 2.53 / 4.7e6 + 1;
+  const double ks = (double)st::cdiv(Q, BK);
+  const int64_t K = NN ? P : Q, cus = cu_count();
+  double fused;
+  if (K % 128) {
+    fused = rounds_us(st::cdiv(M, 128) * st::cdiv(P, 128), cus, 1.25, 1.25, ks);
+  } else {
+    switch (tile_choice(MODE, M, P)) {
+      case 256: {
+        const int64_t n = st::cdiv(M, 256) * st::cdiv(P, 256);
+        fused = split_column(256, M, P) ? ((double)(n / cus) + 0.6) * (1.72 * ks + 5)
+                                        : rounds_us(n, cus, 1.4, 1.72, ks);
+        break;
+      }
+      case 2562:
+        fused = rounds_us(st::cdiv(M, 256) * st::cdiv(P, 128), cus, 0.85, 1.04, ks);
+        break;
+      default: {
+        const double t = NN ? 0.8 : 0.85;
+        fused = rounds_us(st::cdiv(M, 128) * st::cdiv(P, 128), cus, t, t, ks);
+      }
+    }
+  }
+  return dma < fused;
+}
+int64_t decode_workspace(int64_t N, int64_t K) { return N * K * 2 + 256; }
+
+// Decodes W [N, K] into the workspace and runs the GEMM on it (p.ldw = K).
+template <bool NN>
+int decode_and_run(GemmParams p, const uint8_t* payload, const float* scales, int64_t N,
+                   const float* lut16, int32_t flags, void* workspace, hipStream_t stream) {
+  uint16_t* w = (uint16_t*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
+  if (int rc = st::launch_dequant4(payload, scales, N * p.ldw, 1 << p.gshift, lut16, flags, w,
+                                   stream))
+    return rc;
+  p.Wb = w;
+  p.w_bytes = N * p.ldw * 2;
+  // the sums run in the order of the fused kernel that the call would take
+  // without a workspace, so that the workspace does not change the result
+  if constexpr (!NN)
+    if (forward_runs_rb(p)) return launch_dma<false, true>(p, stream);
+  return launch_dma<NN>(p, stream);
+}
 
 }  // namespace
 
-// Every shape runs from the packed weight (K % 128 != 0 on the flat-group
-// kernels), so the fused linears take no workspace; the queries stay for
-// callers that size one.
+// Every shape also runs from the packed weight without a workspace.
 extern "C" int64_t st_q4_linear_fwd_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (decode_first<FWD_Q4>(M, N, K)) return decode_workspace(N, K);
   return split_workspace(split_plan(M, N, K), M, N);
 }
 
 extern "C" int64_t st_q4_linear_dgrad_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
+  if (decode_first<DGRAD_Q4>(M, K, N)) return decode_workspace(N, K);
   return split_workspace(split_plan(M, K, N), M, K);
 }
 
@@ -1749,12 +2089,15 @@ extern "C" int st_q4_linear_fwd(const uint16_t* x, int64_t M, int64_t K, int64_t
   ST_CHECK_ARG(((uintptr_t)payload & 3u) == 0, "st_q4_linear_fwd: payload not 4-byte aligned");
   p.Wq = payload; p.Ws = scales; p.ldw = K;
   p.w_bytes = N * K / 2; p.s_bytes = st::cdiv(N * K, 1ll << p.gshift) * 4;
+  if (workspace && decode_first<FWD_Q4>(M, N, K) && workspace_bytes >= decode_workspace(N, K) &&
+      dma_lora_fits<false>(p))
+    return decode_and_run<false>(p, payload, scales, N, lut16, flags, workspace, s);
   if (K % (1 << p.gshift) == 0 && al16(payload)) {
     // split-K when the caller brought the workspace the query asks for
     const SplitPlan plan = split_plan(M, N, K);
     if (plan.splits > 1 && workspace && workspace_bytes >= split_workspace(plan, M, N))
       return launch_ws_split<FWD_Q4>(p, plan, workspace, s);
-    return run_gemm(FWD_Q4, p, s);
+    return dispatch<FWD_Q4>(p, s);
   }
   // flat scale groups straddle W's rows (or 16-byte loads would be misaligned):
   // per-word scales on the 128x128 tile
@@ -1800,12 +2143,15 @@ static int dgrad_impl(const uint16_t* dy, int64_t M, int64_t N, int64_t lddy,
   ST_CHECK_ARG(((uintptr_t)payload & 3u) == 0, "st_q4_linear_dgrad: payload not 4-byte aligned");
   p.Wq = payload; p.Ws = scales; p.ldw = K;
   p.w_bytes = N * K / 2; p.s_bytes = st::cdiv(N * K, 1ll << p.gshift) * 4;
+  if (workspace && decode_first<DGRAD_Q4>(M, K, N) && workspace_bytes >= decode_workspace(N, K) &&
+      dma_lora_fits<true>(p))
+    return decode_and_run<true>(p, payload, scales, N, lut16, flags, workspace, s);
   if (K % (1 << p.gshift) == 0) {
     // split-K (not with the SwiGLU VJP) when the caller brought the workspace
     const SplitPlan plan = split_plan(M, K, N);
     if (!gu && plan.splits > 1 && workspace && workspace_bytes >= split_workspace(plan, M, K))
       return launch_ws_split<DGRAD_Q4>(p, plan, workspace, s);
-    return run_gemm(DGRAD_Q4, p, s);
+    return dispatch<DGRAD_Q4>(p, s);
   }
   // flat scale groups straddle W's rows: per-word scales on the 128x128 tile
   return launch<DGRAD_Q4, 128, 128, 4, 2, true>(p, s);
@@ -1996,11 +2342,7 @@ extern "C" int st_linear_bf16_fwd(const uint16_t* x, int64_t M, int64_t K, int64
   p.w_bytes = ((N - 1) * ldw + K) * 2;
   ST_CHECK_ARG(p.a_bytes < (1ll << 31) && p.w_bytes < (1ll << 31),
                "st_linear_bf16_fwd: operands above 2 GiB are not supported");
-  // 256x256 tiles where they fill the GPU (the terminal's head GEMM over a
-  // whole sequence), 128x128 otherwise
-  if (st::cdiv(M, 256) * st::cdiv(N, 256) >= 192)
-    return launch<FWD_BF16, 256, 256, 8>(p, (hipStream_t)stream);
-  return launch<FWD_BF16, 128, 128, 4>(p, (hipStream_t)stream);
+  return launch_dma<false>(p, (hipStream_t)stream);
 }
 
 extern "C" int st_linear_bf16_dgrad(const uint16_t* dy, int64_t M, int64_t N, int64_t lddy,
@@ -2020,10 +2362,5 @@ extern "C" int st_linear_bf16_dgrad(const uint16_t* dy, int64_t M, int64_t N, in
   p.w_bytes = ((N - 1) * ldw + K) * 2;
   ST_CHECK_ARG(p.a_bytes < (1ll << 31) && p.w_bytes < (1ll << 31),
                "st_linear_bf16_dgrad: operands above 2 GiB are not supported");
-  // 256x256 tiles where they fill the GPU (measured on the terminal's
-  // [4095, 4096] input gradient over vocab 151936: 256x256 ahead of 256x128,
-  // 128x256 and 128x128), 128x128 otherwise
-  if (st::cdiv(M, 256) * st::cdiv(K, 256) >= 192)
-    return launch<DGRAD_BF16, 256, 256, 8>(p, (hipStream_t)stream);
-  return launch<DGRAD_BF16, 128, 128, 4>(p, (hipStream_t)stream);
+  return launch_dma<true>(p, (hipStream_t)stream);
 }

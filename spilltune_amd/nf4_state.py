@@ -24,7 +24,7 @@ This module takes the same parts:
   copies, staged with ``non_blocking`` copies on a caller's stream and
   converted on the device by ``st_nf4_dq_scales`` into a :class:`ops.Q4Weight`
   whose GEMMs read the packed bytes as they lie (high nibble first,
-  ``ST_FLAG_GROUP64``): W is never written to HBM as bf16.
+  ``ST_FLAG_GROUP64``); no bf16 copy of W outlives a call.
 * :func:`linear_cuda` -- the base linear of nf4_backend_cuda.py:888-917 on
   the fused GEMM (autograd: the input gradient on the fused dgrad GEMM).
 

@@ -204,6 +204,19 @@ class _Workspace:
 _ws = _Workspace()
 
 
+def _gemm_scratch(device, nbytes: int) -> torch.Tensor | None:
+    """Scratch of one fused GEMM call (decoded weights or split-K partials),
+    from the caching allocator, so that it belongs to the current stream.  None
+    when nothing is needed or the device has no room for it: the call then
+    decodes inside the GEMM."""
+    if nbytes <= 0:
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def lora_gemm(Mo, No, Kc, a, sam, sak, b, sbk, sbn, alpha, out, accumulate=False):
     """``out = (accumulate ? out : 0) + alpha * sum_k a(m,k) b(k,n)`` (fp32 out)."""
     need = _lib.query("st_lora_gemm_workspace_bytes", Mo, No, Kc)
@@ -359,8 +372,9 @@ class _Q4LoRALinear(torch.autograd.Function):
             # T = x_f32 A_cat^T   (lora.py:219 inner linear)
             lora_gemm(M, nseg * rank, K, x, K, 1, A_cat, 1, K, 1.0, T)
             ends = _lib.i64_array(torch.tensor(weight.segments).cumsum(0).tolist())
-        # split-K partials for shapes whose tiles leave CUs idle (0 otherwise)
-        ws = _ws.get(dev, _lib.query("st_q4_linear_fwd_workspace_bytes", M, N, K))
+        # W decoded once for many rows, or split-K partials for shapes whose
+        # tiles leave CUs idle (0 otherwise)
+        ws = _gemm_scratch(dev, _lib.query("st_q4_linear_fwd_workspace_bytes", M, N, K))
         _launch(("fwd", M, N, K), lambda: _lib.call(
             "st_q4_linear_fwd", _lib.ptr(x), M, K, K, _lib.ptr(weight.payload),
             _lib.ptr(weight.scales), N, weight.lut(), weight.flags,
@@ -469,13 +483,15 @@ class _Q4LoRALinear(torch.autograd.Function):
         if ctx.swiglu_I:
             # the dgrad epilogue applies the SwiGLU VJP: the gradient of gate|up
             dx = torch.empty_like(gu)
+            ws = _gemm_scratch(dev, _lib.query("st_q4_linear_dgrad_workspace_bytes", M, N, K))
             _launch(("dgrad", M, N, K), lambda: _lib.call(
                 "st_q4_linear_dgrad_swiglu", _lib.ptr(dy), M, N, N, _lib.ptr(weight.payload),
                 _lib.ptr(weight.scales), K, weight.lut(), weight.flags, *lora_args,
-                _lib.ptr(gu), gu.stride(0), _lib.ptr(dx), dx.stride(0), None, 0, stream))
+                _lib.ptr(gu), gu.stride(0), _lib.ptr(dx), dx.stride(0), _lib.ptr(ws),
+                0 if ws is None else ws.numel(), stream))
         else:
             dx = torch.empty((M, K), dtype=_BF16, device=dev)
-            ws = _ws.get(dev, _lib.query("st_q4_linear_dgrad_workspace_bytes", M, N, K))
+            ws = _gemm_scratch(dev, _lib.query("st_q4_linear_dgrad_workspace_bytes", M, N, K))
             _launch(("dgrad", M, N, K), lambda: _lib.call(
                 "st_q4_linear_dgrad", _lib.ptr(dy), M, N, N, _lib.ptr(weight.payload),
                 _lib.ptr(weight.scales), K, weight.lut(), weight.flags, *lora_args,
