@@ -161,6 +161,20 @@ __device__ __forceinline__ void raster(int64_t t, int64_t tiles_m, int64_t tiles
   pt = r / h;
 }
 
+// Tile of workgroup b of a grouped launch, whose row-tile slots past the last
+// group's exit at once: slot mt goes to XCD mt % 8 (its column tiles one after
+// the other there, sharing the group's A rows in that L2), so the empty slots
+// at the end fall on all XCDs alike.  Contiguous runs of slots per XCD left
+// the last XCDs with nothing but empty ones (256 experts of ~64 rows: 384
+// slots of 128 rows, 96 of them on two XCDs without work).  The grid holds a
+// multiple of 8 slots.
+__device__ __forceinline__ void grouped_raster(unsigned b, unsigned tiles_p, int64_t& mt,
+                                               int64_t& pt) {
+  const unsigned i = b / 8;
+  mt = (int64_t)(i / tiles_p) * 8 + b % 8;
+  pt = i % tiles_p;
+}
+
 // Grouped (per-expert) row tiles: group g owns rows [off[g], off[g+1]) and
 // cdiv(rows_g, BM) tiles, numbered consecutively over the groups.  Maps tile
 // `slot` to its group, first row and the group's row end (clamped to `rows`).

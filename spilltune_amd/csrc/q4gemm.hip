@@ -708,9 +708,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_kernel(GemmParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / TL::WAVES_N, wn = wave % TL::WAVES_N;
   const int64_t tiles_p = st::cdiv(p.P, BN);
-  const int64_t t = st::xcd_remap(blockIdx.x, gridDim.x);
   int64_t mt, pt;
-  st::raster(t, st::cdiv(p.M, BM), tiles_p, p.raster_m, mt, pt);
+  if (p.goff)
+    st::grouped_raster(blockIdx.x, (unsigned)tiles_p, mt, pt);
+  else
+    st::raster(st::xcd_remap(blockIdx.x, gridDim.x), st::cdiv(p.M, BM), tiles_p, p.raster_m, mt,
+               pt);
   const int64_t p0 = pt * BN;
   int64_t m0 = mt * BM, mend = p.M;
   int grp = 0;
@@ -1027,7 +1030,10 @@ __global__ __launch_bounds__(512) void gemm_ws_kernel(GemmParams p) {
     qlen = p.Q - q0 < (int64_t)p.ks_len * BK ? p.Q - q0 : (int64_t)p.ks_len * BK;
   }
   int64_t mt, pt;
-  st::raster(t, st::cdiv(p.M, BM), tiles_p, p.raster_m, mt, pt);
+  if (p.goff)
+    st::grouped_raster(blockIdx.x, (unsigned)tiles_p, mt, pt);
+  else
+    st::raster(t, st::cdiv(p.M, BM), tiles_p, p.raster_m, mt, pt);
   const int64_t p0 = pt * BN;
   int64_t m0 = mt * BM, mend = p.M;
   int grp = 0;
@@ -1372,9 +1378,12 @@ __global__ __launch_bounds__(64 * WAVES, FM == 4 ? 4 : 1) void gemm_rb_kernel(Ge
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t tiles_p = st::cdiv(p.P, BN);
-  const int64_t t = st::xcd_remap(blockIdx.x, gridDim.x);
   int64_t mt, pt;
-  st::raster(t, st::cdiv(p.M, BM), tiles_p, p.raster_m, mt, pt);
+  if (p.goff)
+    st::grouped_raster(blockIdx.x, (unsigned)tiles_p, mt, pt);
+  else
+    st::raster(st::xcd_remap(blockIdx.x, gridDim.x), st::cdiv(p.M, BM), tiles_p, p.raster_m, mt,
+               pt);
   const int64_t p0 = pt * BN;
   int64_t m0 = mt * BM, mend = p.M;
   int grp = 0;
@@ -1596,10 +1605,11 @@ int raster_choice(const GemmParams& p) {
 }
 
 // Row-tile slots of a launch: grouped launches (per-expert row ranges) take
-// sum_g cdiv(rows_g, BM) <= cdiv(rows, BM) + groups; slots past the last
-// group's tiles exit at once.
+// sum_g cdiv(rows_g, BM) <= cdiv(rows, BM) + groups, a multiple of 8 for
+// st::grouped_raster; slots past the last group's tiles exit at once.
 int64_t row_tiles(const GemmParams& p, int BM) {
-  return st::cdiv(p.M, BM) + (p.goff ? p.ngroups : 0);
+  const int64_t n = st::cdiv(p.M, BM);
+  return p.goff ? st::cdiv(n + p.ngroups, 8) * 8 : n;
 }
 
 // The epilogue addresses C, the residual, T and the LoRA right operand with
