@@ -89,18 +89,20 @@ class Q4Weight:
 MAX_LORA_COLS = 64  # LoRA columns (segments x rank) one fused GEMM epilogue stages
 
 
-def lora_fusable(loras) -> bool:
+def lora_fusable(loras, partial: bool = False) -> bool:
     """Whether N-concatenated projections with these adapters can run as one
-    fused GEMM: no adapter at all, or one on every part with a single rank and
-    scale and at most MAX_LORA_COLS LoRA columns in all (the epilogue's
-    limit).  Otherwise callers run the projections one by one."""
+    fused GEMM: no adapter at all, or one on every part (``partial``: on some
+    of them) with a single rank and scale and at most MAX_LORA_COLS LoRA
+    columns in all (the epilogue's limit).  Otherwise callers run the
+    projections one by one."""
     loras = list(loras)
-    if all(l is None for l in loras):
+    present = [l for l in loras if l is not None]
+    if not present:
         return True
-    if any(l is None for l in loras):
+    if len(present) < len(loras) and not partial:
         return False
-    ranks = {int(l.rank) for l in loras}
-    scales = {float(l.scale) for l in loras}
+    ranks = {int(l.rank) for l in present}
+    scales = {float(l.scale) for l in present}
     return len(ranks) == 1 and len(scales) == 1 and len(loras) * ranks.pop() <= MAX_LORA_COLS
 
 
@@ -315,14 +317,15 @@ def _rk(G, ldg, S, ssk, big, r, Kc, alpha, out, so_m, so_j, accumulate):
 
 
 # ----------------------------------------------------------------- projection
-def _lora_meta(weight: Q4Weight, loras):
+def _lora_meta(weight: Q4Weight, loras, partial: bool):
     loras = list(loras) if loras is not None else []
-    if not loras or all(l is None for l in loras):
+    present = [l for l in loras if l is not None]
+    if not present:
         return None
-    if len(loras) != len(weight.segments) or any(l is None for l in loras):
+    if len(loras) != len(weight.segments) or (len(present) < len(loras) and not partial):
         raise ValueError("unsupported_capability: fused projections need a LoRA on every segment")
-    ranks = {int(l.rank) for l in loras}
-    scales = {float(l.scale) for l in loras}
+    ranks = {int(l.rank) for l in present}
+    scales = {float(l.scale) for l in present}
     if len(ranks) != 1 or len(scales) != 1:
         raise ValueError("unsupported_capability: fused projections need one rank and scale")
     return ranks.pop(), scales.pop()
@@ -414,7 +417,8 @@ class _Q4LoRALinear(torch.autograd.Function):
             for width in weight.segments:
                 starts.append(starts[-1] + width)
             if sink is not None and not (
-                    ctx.loras is not None and rank <= 64 and all(sink.wants(l) for l in ctx.loras)
+                    ctx.loras is not None and rank <= 64
+                    and all(l is None or sink.wants(l) for l in ctx.loras)
                     and all(st % 8 == 0 for st in starts) and N % 8 == 0 and K % 8 == 0
                     and dy.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0):
                 sink = None
@@ -435,6 +439,8 @@ class _Q4LoRALinear(torch.autograd.Function):
                               dT[:, s_ * rank:(s_ + 1) * rank])
             acc = sink.accumulate
             for s_, lo in enumerate(ctx.loras):
+                if lo is None:
+                    continue
                 off, width = starts[s_], weight.segments[s_]
                 Ts, dTs = T[:, s_ * rank:], dT[:, s_ * rank:]
                 sink.add(lo, [
@@ -500,12 +506,28 @@ class _Q4LoRALinear(torch.autograd.Function):
         return (dx, None, dres, None, None, None, None, *grads_ab)
 
 
+def _fill_loras(weight: Q4Weight, loras, rank: int, device):
+    """``(A, B)`` of every segment, zeros (one buffer for all) where a segment
+    has no adapter: its T columns are zero and its outputs the plain base."""
+    missing = [n for n, l in zip(weight.segments, loras) if l is None]
+    if missing:
+        K = weight.in_features
+        zeros = torch.zeros(rank * max(K, *missing), dtype=_F32, device=device)
+    ab = []
+    for n, l in zip(weight.segments, loras):
+        ab += [zeros[:rank * K].view(rank, K), zeros[:n * rank].view(n, rank)] if l is None \
+            else [l.A, l.B]
+    return ab
+
+
 def q4_lora_linear(x: torch.Tensor, weight: Q4Weight, loras=None, residual=None,
-                   swiglu: bool = False) -> torch.Tensor:
+                   swiglu: bool = False, partial: bool = False) -> torch.Tensor:
     """``bf16(bf16(x W^T) + s (x_f32 A^T) B^T)`` [``+ residual``] for a 2-D bf16 ``x``.
 
     ``loras`` holds one LoRA object (``A``, ``B``, ``rank``, ``scale``) per
-    segment of ``weight`` or is None.  ``swiglu``: ``x`` is a fused gate|up
+    segment of ``weight`` or is None; with ``partial`` some of a fused weight's
+    segments may have None (the reference adapts q, v and o by default): they
+    still run as one GEMM.  ``swiglu``: ``x`` is a fused gate|up
     pre-activation ``[M, 2I]`` and the projection reads ``silu(gate) * up``
     (dense.py:153); the backward applies the SwiGLU VJP inside the input-
     gradient GEMM and returns the gradient of gate|up."""
@@ -517,7 +539,7 @@ def q4_lora_linear(x: torch.Tensor, weight: Q4Weight, loras=None, residual=None,
                          f"{weight.in_features}{' (gate|up)' if swiglu else ''}")
     x = x.contiguous()
     swiglu_I = width if swiglu else 0
-    meta = _lora_meta(weight, loras)
+    meta = _lora_meta(weight, loras, partial)
     if residual is not None:
         residual = residual.contiguous()
         if residual.shape != (x.shape[0], weight.out_features) or residual.dtype != _BF16:
@@ -525,10 +547,9 @@ def q4_lora_linear(x: torch.Tensor, weight: Q4Weight, loras=None, residual=None,
     if meta is None:
         return _Q4LoRALinear.apply(x, weight, residual, 0, 1.0, swiglu_I, None)
     rank, scale = meta
-    ab = [t for l in loras for t in (l.A, l.B)]
-    for l in loras:
-        if l.A.dtype != _F32 or l.B.dtype != _F32:
-            raise ValueError("LoRA A/B must be fp32")
+    ab = _fill_loras(weight, loras, rank, x.device)
+    if any(t.dtype != _F32 for t in ab):
+        raise ValueError("LoRA A/B must be fp32")
     return _Q4LoRALinear.apply(x, weight, residual, rank, scale, swiglu_I, tuple(loras), *ab)
 
 
