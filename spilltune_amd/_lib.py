@@ -9,6 +9,7 @@ for argument/capability errors, ``RuntimeError`` for device failures.
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from pathlib import Path
 
@@ -153,11 +154,17 @@ def query(name: str, *args) -> int:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def stream_handle(device: torch.device | None = None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def stream_handle(device: torch.device | None = None) -> int:
+    """The current stream's handle (an int, as every pointer argument takes)
+    without building a Stream object: a layer step asks for it ~40 times."""
+    if device is not None and device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
+    index = device.index if device is not None else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None
+                                              else index)
 
 
 class RkProduct(ctypes.Structure):
@@ -169,9 +176,14 @@ class RkProduct(ctypes.Structure):
                 ("so_j", ctypes.c_int64), ("accumulate", ctypes.c_int32)]
 
 
+@functools.lru_cache(maxsize=16)
+def _lut(values: tuple) -> ctypes.Array:
+    return (ctypes.c_float * 16)(*values)
+
+
 def lut_array(values) -> ctypes.Array:
-    arr = (ctypes.c_float * 16)(*[float(v) for v in values])
-    return arr
+    """16 floats for the C ABI (read only; the codebooks' are made once)."""
+    return _lut(tuple(float(v) for v in values))
 
 
 def i64_array(values) -> ctypes.Array:

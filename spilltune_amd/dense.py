@@ -103,8 +103,9 @@ def dense_block(hidden_states, position_embeddings, attention_mask, *, heads, kv
     qkv = ops.concat_rows([wq, wk, wv])
     loras_qkv = [lora_q, lora_k, lora_v]
     # adapters on some of q, k and v (q, v, o by default) still run as one GEMM:
-    # one after the other, k and v alone are too narrow to fill the GPU (three
-    # rows of 701 tokens, 4096 wide: three products 174 us against 95)
+    # one after the other, k and v alone are too narrow to fill the GPU (2103
+    # rows, 4096 wide: 99 + 74 + 74 us a pass against 95 in one, besides the
+    # separate head norms, rotations and gradient adds: a step of 3.81 -> 3.38 ms)
     if qkv is not None and ops.lora_fusable(loras_qkv, partial=True):
         y = ops.q4_lora_linear(xn, qkv, loras_qkv, partial=True)
         if qk_norm:

@@ -24,6 +24,7 @@ import math
 from contextlib import contextmanager
 
 from dataclasses import dataclass, field
+from itertools import accumulate
 
 import torch
 
@@ -374,7 +375,7 @@ class _Q4LoRALinear(torch.autograd.Function):
             T = torch.empty((M, nseg * rank), dtype=_F32, device=dev)
             # T = x_f32 A_cat^T   (lora.py:219 inner linear)
             lora_gemm(M, nseg * rank, K, x, K, 1, A_cat, 1, K, 1.0, T)
-            ends = _lib.i64_array(torch.tensor(weight.segments).cumsum(0).tolist())
+            ends = _lib.i64_array(list(accumulate(weight.segments)))
         # W decoded once for many rows, or split-K partials for shapes whose
         # tiles leave CUs idle (0 otherwise)
         ws = _gemm_scratch(dev, _lib.query("st_q4_linear_fwd_workspace_bytes", M, N, K))
@@ -455,7 +456,7 @@ class _Q4LoRALinear(torch.autograd.Function):
             dB_all = torch.empty((N, rank), dtype=_F32, device=dev)
             # dT_s = s * dY_s B_s and dB_s = s * dY_s^T T_s for every segment:
             # one launch of partial products and one reduction
-            ends = _lib.i64_array(torch.tensor(weight.segments).cumsum(0).tolist())
+            ends = _lib.i64_array(list(accumulate(weight.segments)))
             need = _lib.query("st_lora_bwd_dy_workspace_bytes", M, N, rank, nseg, ends)
             if need > 0:
                 ws = _ws.get(dev, need)
