@@ -1363,8 +1363,10 @@ __device__ __forceinline__ void rb_order() {
   }
 }
 #undef RB_G
-template <int FN, int WAVES, bool HI, int FM = 8>
-__global__ __launch_bounds__(64 * WAVES, FM == 4 ? 4 : 1) void gemm_rb_kernel(GemmParams p) {
+// rows [m0, m0 + 32*FM) of group grp (those before mend), columns from p0
+template <int FN, int WAVES, bool HI, int FM>
+__device__ __forceinline__ void rb_tile(const GemmParams& p, uint4* ldsA, int grp, int64_t m0,
+                                        int64_t mend, int64_t p0) {
   constexpr int BM = 32 * FM, NT = 64 * WAVES, WN = 32 * FN, BN = WN * WAVES;
   constexpr int WM = BM;
   constexpr int A_ST = BM * BK / 8;       // 16-byte units per A stage
@@ -1373,23 +1375,9 @@ __global__ __launch_bounds__(64 * WAVES, FM == 4 ? 4 : 1) void gemm_rb_kernel(Ge
   // scale loads for a tile that starts a scale group (even tiles); two
   // consecutive steps issue RB_PAIR of them
   constexpr int RB_PAIR = 2 * DMA_W + 3 * FN;
-  __shared__ uint4 ldsA[RB_ST * A_ST];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t tiles_p = st::cdiv(p.P, BN);
-  int64_t mt, pt;
-  if (p.goff)
-    st::grouped_raster(blockIdx.x, (unsigned)tiles_p, mt, pt);
-  else
-    st::raster(st::xcd_remap(blockIdx.x, gridDim.x), st::cdiv(p.M, BM), tiles_p, p.raster_m, mt,
-               pt);
-  const int64_t p0 = pt * BN;
-  int64_t m0 = mt * BM, mend = p.M;
-  int grp = 0;
-  if (p.goff) {  // grouped (per-expert) rows: the whole workgroup leaves together
-    if (!st::find_group(p.goff, p.ngroups, BM, mt, p.M, grp, m0, mend)) return;
-  }
   const int KT = (int)(p.Q / BK);
   const auto rsA = make_rsrc(p.A, p.a_bytes);
   const auto rsW = make_rsrc(p.Wq + grp * p.w_gstride, p.w_bytes);
@@ -1539,6 +1527,39 @@ __global__ __launch_bounds__(64 * WAVES, FM == 4 ? 4 : 1) void gemm_rb_kernel(Ge
   __syncthreads();
   gemm_epilogue<false, BM, BN, NT, FM, FN, WM, WN>(p, acc, ldsA, m0, mend, p0, 0, wave, tid, lane,
                                                    true, p.L + grp * p.l_gstride);
+}
+
+template <int FN, int WAVES, bool HI, int FM = 8>
+__global__ __launch_bounds__(64 * WAVES, FM == 4 ? 4 : 1) void gemm_rb_kernel(GemmParams p) {
+  constexpr int BM = 32 * FM, BN = 32 * FN * WAVES;
+  __shared__ uint4 ldsA[RB_ST * BM * BK / 8];
+  const int64_t tiles_p = st::cdiv(p.P, BN);
+  int64_t mt, pt;
+  if (p.goff)
+    st::grouped_raster(blockIdx.x, (unsigned)tiles_p, mt, pt);
+  else
+    st::raster(st::xcd_remap(blockIdx.x, gridDim.x), st::cdiv(p.M, BM), tiles_p, p.raster_m, mt,
+               pt);
+  int64_t m0 = mt * BM, mend = p.M;
+  int grp = 0;
+  if (p.goff) {  // grouped (per-expert) rows: the whole workgroup leaves together
+    if (!st::find_group(p.goff, p.ngroups, BM, mt, p.M, grp, m0, mend)) return;
+  }
+  // The 128-row tile of experts with few rows: the last tile of an expert with
+  // at most 64 rows left runs the 64-row body, half the products and half the
+  // LDS reads (per 64 x 256 x 64 step the products take as long as the decode;
+  // neither hides wholly under the loads of W).  Each output keeps its sums
+  // and their order.  64-row slots for all would read and decode W twice for
+  // every expert with more.  256 experts of ~64 rows (half of them with at
+  // most 64), 7168 -> 4096: 2173 -> 2036 us, 2048 -> 7168: 1032 -> 951 us; 128
+  // experts of ~256 rows, 2048 -> 1536: 274 -> 270 us.
+  if constexpr (FM == 4) {
+    if (mend - m0 <= BM / 2) {
+      rb_tile<FN, WAVES, HI, FM / 2>(p, ldsA, grp, m0, mend, pt * BN);
+      return;
+    }
+  }
+  rb_tile<FN, WAVES, HI, FM>(p, ldsA, grp, m0, mend, pt * BN);
 }
 
 // bf16 x bf16 GEMM with both operands moved by DMA (gemm_dma.h): the plain

@@ -54,3 +54,30 @@ def test_grouped_gemms_over_uneven_groups(rows, N, K, hi_first):
             slack = (a.abs() @ b.abs()) / a.shape[1] ** 0.5
             ref = a @ b
             assert ((got.float() - ref).abs() <= 2 ** -8 * (ref.abs() + slack)).all(), (e, n)
+
+
+def test_half_row_tiles_equal_the_256_row_tile(monkeypatch):
+    """Expert tails of at most 64 rows take half a 128-row tile: the same sums,
+    adapters included, as the 256-row tile (bit for bit), on odd columns."""
+    dev, rows, N, K, r = torch.device("cuda:0"), [1, 63, 64, 65, 128, 129, 192, 193, 300], 328, 512, 8
+    g = torch.Generator(device=dev).manual_seed(5)
+    E, R = len(rows), sum(rows)
+    q = moe.Q4Experts(
+        torch.randint(0, 256, (E * N * K // 2,), dtype=torch.uint8, device=dev, generator=g),
+        torch.rand(E * N * K // 128, device=dev, generator=g) * 0.03 + 0.01, E, N, K, "nf4-g128")
+    off = torch.tensor([0] + rows, device=dev).cumsum(0).int()
+    x = torch.randn(R, K, device=dev, generator=g).to(BF)
+    T = torch.randn(R, r, device=dev, generator=g)
+    B = torch.randn(E, N, r, device=dev, generator=g) * 0.1
+    P, got = _lib.ptr, []
+    for tile in ("2568", "2566"):
+        monkeypatch.setenv("ST_GROUPED_TILE", tile)
+        for lora in (False, True):
+            y = torch.full((R, N), 7.0, dtype=BF, device=dev)
+            args = (P(T), r, P(B), r, 0.5, 1, _lib.i64_array([N])) if lora else \
+                (None, 0, None, 0, 1.0, 0, None)
+            _lib.call("st_q4_grouped_fwd", P(x), R, K, None, R, K, P(off), E, P(q.payload),
+                      P(q.scales), N, q.lut(), 0, *args, P(y), N, _lib.stream_handle(dev))
+            got.append(y)
+    assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[3])
+    assert not torch.equal(got[0], got[1])
