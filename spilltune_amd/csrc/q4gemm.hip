@@ -6,8 +6,9 @@
 // Generic form inside the kernel: C[M,P] = A[M,Q] * B[Q,P], Q = contraction.
 // The packed weight is streamed from HBM (0.53 B/element), dequantised in
 // registers (codebook in LDS, one fp32 multiply + RNE per element, the exact
-// arithmetic of codecs.py:168-170) and written to LDS as bf16, so W never
-// exists in HBM as bf16.  The A tile and the forward B tile are stored
+// arithmetic of codecs.py:168-170) and written to LDS as bf16.  With many rows
+// W is decoded once into the caller's workspace instead and the bf16 DMA tiles
+// of gemm_dma.h run (decode_first says when).  The A tile and the forward B tile are stored
 // contraction-contiguous in padded 144-byte rows; the dgrad B tile keeps W's
 // natural [contraction][output] orientation and its MFMA operand is read with
 // the transposing ds_read_b64_tr_b16.
