@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import threading
+from array import array
 from pathlib import Path
 
 import torch
@@ -177,13 +178,14 @@ class RkProduct(ctypes.Structure):
 
 
 @functools.lru_cache(maxsize=16)
-def _lut(values: tuple) -> ctypes.Array:
-    return (ctypes.c_float * 16)(*values)
+def _lut(packed: bytes) -> ctypes.Array:
+    return (ctypes.c_float * 16)(*array("d", packed))
 
 
 def lut_array(values) -> ctypes.Array:
-    """16 floats for the C ABI (read only; the codebooks' are made once)."""
-    return _lut(tuple(float(v) for v in values))
+    """16 floats for the C ABI (read only; the codebooks' are made once, found
+    by their bits: as numbers 0.0 and -0.0 are equal, their codes are not)."""
+    return _lut(array("d", map(float, values)).tobytes())
 
 
 def i64_array(values) -> ctypes.Array:

@@ -45,6 +45,16 @@ def test_abi_version_and_error_mapping():
                   1, 1, 1.0, ctypes.c_void_p(16), 4, 0, None, 0, None)
 
 
+def test_lut_array_keeps_the_sign_of_zero():
+    """Codebooks that are equal as numbers but not in their bits each get
+    their own table, in either order; equal bits share one."""
+    pos = [0.0] + [0.5] * 15
+    neg = [-0.0] + [0.5] * 15
+    for values, sign in ((pos, "0000"), (neg, "8000"), (pos, "0000")):
+        assert bytes(_lib.lut_array(values))[:4][::-1].hex() == sign + "0000"
+    assert bytes(_lib.lut_array(range(16))) == bytes((ctypes.c_float * 16)(*range(16)))
+
+
 def test_lora_rank_limits_rejected_before_any_launch():
     """Rank bounds of the LoRA entry points: checked on the host, before any
     device work (fake pointers never reach a kernel)."""
