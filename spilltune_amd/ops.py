@@ -351,6 +351,15 @@ def _stack_rows(ts):
     return t0.as_strided((rows, width), (width, 1), t0.storage_offset())
 
 
+def _clear_missing(t, loras, rank: int) -> None:
+    """Zeros in the LoRA columns of the segments without an adapter.  Their zero
+    factors give zeros for finite rows only (0 * inf is NaN), and such a segment
+    has no adapter term that could turn its infinities into NaN."""
+    for s, l in enumerate(loras or ()):
+        if l is None:
+            t[:, s * rank:(s + 1) * rank].zero_()
+
+
 class _Q4LoRALinear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, residual, rank, scale, swiglu_I, loras, *ab):
@@ -375,6 +384,7 @@ class _Q4LoRALinear(torch.autograd.Function):
             T = torch.empty((M, nseg * rank), dtype=_F32, device=dev)
             # T = x_f32 A_cat^T   (lora.py:219 inner linear)
             lora_gemm(M, nseg * rank, K, x, K, 1, A_cat, 1, K, 1.0, T)
+            _clear_missing(T, loras, rank)
             ends = _lib.i64_array(list(accumulate(weight.segments)))
         # W decoded once for many rows, or split-K partials for shapes whose
         # tiles leave CUs idle (0 otherwise)
@@ -485,6 +495,8 @@ class _Q4LoRALinear(torch.autograd.Function):
                 grads_ab += [dA_cat[s * rank:(s + 1) * rank], dBs[s]]
         else:
             x, gu = ctx.saved_tensors
+        if dT is not None:
+            _clear_missing(dT, ctx.loras, rank)
         lora_args = (_lib.ptr(dT), 0 if dT is None else dT.stride(0), _lib.ptr(A_cat),
                      0 if dT is None else dT.shape[1])
         if ctx.swiglu_I:
@@ -509,7 +521,8 @@ class _Q4LoRALinear(torch.autograd.Function):
 
 def _fill_loras(weight: Q4Weight, loras, rank: int, device):
     """``(A, B)`` of every segment, zeros (one buffer for all) where a segment
-    has no adapter: its T columns are zero and its outputs the plain base."""
+    has no adapter (its LoRA columns are cleared, _clear_missing): its outputs
+    are the plain base."""
     missing = [n for n, l in zip(weight.segments, loras) if l is None]
     if missing:
         K = weight.in_features

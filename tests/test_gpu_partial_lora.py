@@ -61,3 +61,38 @@ def test_partial_adapters_equal_separate_projections(M, rank, has, deferred):
     assert torch.allclose(got[0].float(), want[0].float(), rtol=2 ** -6, atol=2 ** -6 * want[0].float().abs().mean().item() * 4)
     for a, b in zip(got[1:], want[1:]):  # fp32 sums of the same products
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-4 * b.abs().max().item())
+
+
+@pytest.mark.parametrize("has", [(1, 0, 1), (0, 1, 0)])
+def test_infinite_rows_stay_infinite_without_an_adapter(has):
+    """An infinity in a row of x (or dY) makes that row's outputs (or input
+    gradient) infinite, not NaN, in the segments without an adapter: they have
+    no adapter term.  The weights hold no zeros (0 * inf is NaN by itself)."""
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(11)
+    M, K, rank, widths = 40, 256, 4, (64, 32, 64)
+    N = sum(widths)
+    nibble = torch.randint(8, 16, (2, N * K // 2), dtype=torch.uint8, device=dev, generator=g)
+    w = ops.Q4Weight(nibble[0] | nibble[1] << 4,  # codes 8..15: positive weights
+                     torch.full((N * K // 128,), 0.02, device=dev), (N, K), "nf4-g128", widths)
+    x = torch.randn(M, K, device=dev, generator=g).to(BF)
+    dy = torch.randn(M, N, device=dev, generator=g).to(BF)
+    x[7, 3] = float("inf")
+    loras = [_L(g, rank, K, n, dev) if h else None for n, h in zip(widths, has)]
+    col = 0
+    for n, h in zip(widths, has):
+        if not h:
+            dy[9, col] = float("-inf")
+        col += n
+    xg = x.clone().requires_grad_(True)
+    y = ops.q4_lora_linear(xg, w, loras, partial=True)
+    (dx,) = torch.autograd.grad(y, [xg], dy)
+    base = ops.q4_lora_linear(x, w, None)
+    col = 0
+    for n, h in zip(widths, has):
+        if not h:
+            assert torch.equal(y[:, col:col + n], base[:, col:col + n])
+            assert (y[7, col:col + n] == float("inf")).all()
+        col += n
+    rest = torch.arange(M, device=dev) != 9
+    assert (dx[9] == float("-inf")).all() and torch.isfinite(dx[rest]).all()
