@@ -272,8 +272,9 @@ struct DmaLoop256 {
 // (64 WM) x (64 WN) tile of 64x64 wave tiles, ST slots of a whole k-step, one
 // phase of 16 MFMAs per 32-deep slice, one barrier per k-step before its last
 // phase.  <4, 2, 3>: 256x128, one workgroup per CU.  <2, 2, 2>: 128x128, two
-// workgroups per CU, each with 64 KiB.  With three slots B's DMAs go out in
-// the first phase and A's in the second (3-5% faster than both behind the
+// workgroups per CU, each with 64 KiB.  <2, 2, 4>: 128x128 alone on a CU with
+// two more steps in flight.  With three slots or more B's DMAs go out in the
+// first phase and A's in the second (3-5% faster than both behind the
 // barrier); with two there is no step to spare and both follow the barrier.
 template <bool NN, bool PERM, int WMS, int WNS, int ST>
 struct DmaLoop64 {

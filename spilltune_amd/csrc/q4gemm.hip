@@ -1914,7 +1914,7 @@ int dispatch(const GemmParams& p, hipStream_t stream) {
 }
 
 // ---- bf16 GEMM on the DMA tiles
-enum DmaKind { DMA_256 = 256, DMA_256x128 = 2561, DMA_128 = 128 };
+enum DmaKind { DMA_256 = 256, DMA_256x128 = 2561, DMA_128 = 128, DMA_128_DEEP = 1284 };
 
 template <class LP>
 int launch_dma_tile(GemmParams p, hipStream_t stream) {
@@ -1943,7 +1943,14 @@ double rounds_us(int64_t n, int64_t slots, double lo, double hi, double ks) {
 // the clock drops (2048 x 4096 x 4096 79 us, 4096 x 4096 x 4096 98); 256x128
 // 0.68 to 0.83 (0.72 to 0.88; 2048 x 4096 x 4096 58 us); a pair of 128x128
 // tiles on a CU 0.7 to 0.87, one alone 0.63 (512 x 4096 x 4096 47 us).
-// ST_GEMM_DMA = 256, 2561 or 128 pins a tile for the tests.
+// A lone 128x128 tile over a long contraction waits for memory with its two
+// slots (a vocabulary's rows: nothing of W is in a cache), so from 256 k-steps
+// it takes four: 0.5 to 0.56.  dX of a 152064-row head, hidden 4096: 64 rows
+// 1901 -> 1213 us, 256 rows 2068 -> 1348, 1024 rows 2000 -> 1319; 32000 rows,
+// 64 rows 321 -> 261.  Operands that stay in L2 gain nothing and pay for the
+// longer prologue (500 x 256 x 7168 forward 57 -> 60 us, 500 x 2048 x 128 6.5
+// -> 7.3), hence the line at 256.
+// ST_GEMM_DMA = 256, 2561, 128 or 1284 pins a tile for the tests.
 DmaKind dma_kind(bool nn, int64_t M, int64_t P, int64_t Q, double* us = nullptr) {
   const double ks = (double)st::cdiv(Q, BK);
   const int64_t cus = cu_count(), n128 = st::cdiv(M, 128) * st::cdiv(P, 128);
@@ -1951,16 +1958,18 @@ DmaKind dma_kind(bool nn, int64_t M, int64_t P, int64_t Q, double* us = nullptr)
                                 nn ? 1.5 : 1.45, ks);
   const double c2561 = rounds_us(st::cdiv(M, 256) * st::cdiv(P, 128), cus, nn ? 0.72 : 0.68,
                                  nn ? 0.88 : 0.83, ks);
-  const double c128 = n128 <= cus ? (nn ? 0.68 : 0.63) * ks + 5
+  const bool deep = n128 <= cus && ks >= 256;
+  const double c128 = deep ? (nn ? 0.56 : 0.55) * ks + 5
+                      : n128 <= cus ? (nn ? 0.68 : 0.63) * ks + 5
                                   : rounds_us(n128, 2 * cus, nn ? 0.72 : 0.7, nn ? 0.92 : 0.87, ks);
   DmaKind k = DMA_256;
   double c = c256;
   if (c2561 < c) c = c2561, k = DMA_256x128;
-  if (c128 < c) c = c128, k = DMA_128;
+  if (c128 < c) c = c128, k = deep ? DMA_128_DEEP : DMA_128;
   if (us) *us = c;
   const char* env = getenv("ST_GEMM_DMA");
   const int e = env ? atoi(env) : 0;
-  return e == DMA_256 || e == DMA_256x128 || e == DMA_128 ? (DmaKind)e : k;
+  return e == DMA_256 || e == DMA_256x128 || e == DMA_128 || e == DMA_128_DEEP ? (DmaKind)e : k;
 }
 
 // PERM: the contraction order of the register-operand forward (gemm_dma.h)
@@ -1969,6 +1978,7 @@ int launch_dma(const GemmParams& p, hipStream_t stream) {
   switch (dma_kind(NN, p.M, p.P, p.Q)) {
     case DMA_256: return launch_dma_tile<st::DmaLoop256<NN, PERM>>(p, stream);
     case DMA_256x128: return launch_dma_tile<st::DmaLoop64<NN, PERM, 4, 2, 3>>(p, stream);
+    case DMA_128_DEEP: return launch_dma_tile<st::DmaLoop64<NN, PERM, 2, 2, 4>>(p, stream);
     default: return launch_dma_tile<st::DmaLoop64<NN, PERM, 2, 2, 2>>(p, stream);
   }
 }
@@ -1981,6 +1991,8 @@ bool dma_lora_fits(const GemmParams& p) {
       return lora_staged_fits<NN, 256, 256>(p, (int64_t)st::DmaLoop256<NN, false>::LDS16 * 4, 8);
     case DMA_256x128:
       return lora_staged_fits<NN, 256, 128>(p, (int64_t)st::DmaLoop64<NN, false, 4, 2, 3>::LDS16 * 4, 8);
+    case DMA_128_DEEP:
+      return lora_staged_fits<NN, 128, 128>(p, (int64_t)st::DmaLoop64<NN, false, 2, 2, 4>::LDS16 * 4, 4);
     default:
       return lora_staged_fits<NN, 128, 128>(p, (int64_t)st::DmaLoop64<NN, false, 2, 2, 2>::LDS16 * 4, 4);
   }

@@ -13,7 +13,7 @@ from spilltune_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
-TILES = ("256", "2561", "128")
+TILES = ("256", "2561", "128", "1284")
 
 
 @pytest.fixture()
@@ -47,6 +47,19 @@ def test_bf16_linear_tiles(dev, monkeypatch, tile, M, N, K):
     x, w, dy = _rand(g, M, K), _rand(g, N, K), _rand(g, M, N)
     _close(ops.linear_bf16(x, w), x, w.t())
     _close(ops.linear_bf16_dgrad(dy, w), dy, w)
+
+
+def test_long_contraction_on_few_tiles(dev, monkeypatch):
+    """The input gradient of a few rows over many (the terminal's short chunks)
+    takes the deeper ring by itself; every tile sums in the same order."""
+    g = torch.Generator(device=dev).manual_seed(8)
+    M, N, K = 130, 256 * 64 + 8, 264
+    w, dy = _rand(g, N, K, scale=0.02), _rand(g, M, N)
+    got = ops.linear_bf16_dgrad(dy, w)
+    _close(got, dy, w)
+    for tile in TILES:
+        monkeypatch.setenv("ST_GEMM_DMA", tile)
+        assert torch.equal(ops.linear_bf16_dgrad(dy, w), got), tile
 
 
 @pytest.mark.parametrize("tile", TILES)
