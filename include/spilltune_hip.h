@@ -100,7 +100,8 @@ int st_nf4_dq_scales(const uint8_t* absmax_q, const float* nested_absmax, const 
  *   y[m,n]    = bf16( residual[m,n] + y[m,n] )            (if residual)
  * W [N,K] is payload/scales in flat groups of 128 (64 with ST_FLAG_GROUP64:
  * bitsandbytes' NF4 blocksize, scales from st_nf4_dq_scales).  K % 8 == 0.
- * `workspace`: the query returns the bytes a shape is fastest with, one of
+ * `workspace`: st_q4_linear_workspace_bytes returns the bytes the call is
+ * fastest with, one of
  *  - 2 N K + 256: many rows; W is decoded to bf16 there once and a bf16 GEMM
  *    runs on it (the fused kernels decode each W panel once per row tile);
  *  - split-K partials (fp32 [splits, M, N], summed in split order by a second
@@ -120,6 +121,18 @@ int st_nf4_dq_scales(const uint8_t* absmax_q, const float* nested_absmax, const 
  * column n belongs to segment s = #{seg_end[i] <= n}; segment ends must be
  * multiples of 32.  nseg = 1 with seg_end[0] = N for a single projection.
  */
+/*
+ * Workspace query of the three forms below: M, N, K and flags as in the call,
+ * rank = LoRA contraction (fwd: rank, dgrads: lora_k; 0: no LoRA), lora_cols =
+ * columns of t (fwd: nseg * rank, dgrads: lora_k).  A decode that would take
+ * more than max_decode_bytes (>= 0) is not asked for.  The call takes the same
+ * path as the query whenever the workspace holds what the query returned.
+ * st_q4_linear_{fwd,dgrad}_workspace_bytes: the same for 128-element groups
+ * without LoRA and without a limit.
+ */
+enum { ST_Q4_FWD = 0, ST_Q4_DGRAD = 1, ST_Q4_DGRAD_SWIGLU = 2 };
+int64_t st_q4_linear_workspace_bytes(int32_t form, int64_t M, int64_t N, int64_t K, int32_t flags,
+                                     int32_t rank, int64_t lora_cols, int64_t max_decode_bytes);
 int64_t st_q4_linear_fwd_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int st_q4_linear_fwd(const uint16_t* x, int64_t M, int64_t K, int64_t ldx,
                      const uint8_t* payload, const float* scales, int64_t N,
@@ -155,7 +168,7 @@ int st_q4_linear_dgrad(const uint16_t* dy, int64_t M, int64_t N, int64_t lddy,
  * dgu[m, I + i] = dup (row stride lddgu).  I is this projection's in_features.
  * gu and dgu must be 16-byte aligned with ldgu, lddgu and I multiples of 8
  * (ST_EUNSUPPORTED otherwise).  `workspace` as for st_q4_linear_dgrad with
- * K = I, split-K aside.
+ * K = I, but never split-K partials.
  */
 int st_q4_linear_dgrad_swiglu(const uint16_t* dy, int64_t M, int64_t N, int64_t lddy,
                               const uint8_t* payload, const float* scales, int64_t I,

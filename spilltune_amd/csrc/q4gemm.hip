@@ -1927,55 +1927,87 @@ int launch_dma_tile(GemmParams p, hipStream_t stream) {
   return st::check_launch("gemm_dma");
 }
 
-// Modelled microseconds of `n` tiles on `slots` at once: whole rounds of `hi`
-// per 64-deep k-step, a last round between `lo` and `hi` with its fill.
-double rounds_us(int64_t n, int64_t slots, double lo, double hi, double ks) {
-  const int64_t rest = n % slots;
-  const double occ = (double)rest / (double)slots;
-  return (double)(n / slots) * (hi * ks + 5) +
-         (rest ? (lo + (hi - lo) * occ * occ * occ) * ks + 5 : 0);
+// Modelled microseconds of a GEMM of `n` tiles: the cost of a 64-deep k-step
+// of a round, from a nearly idle chip (lo) to a full one (hi, where the clock
+// drops), and a tile's fill (with its epilogue: per LoRA rank, and with the
+// SwiGLU VJP).  Tiles of which a CU takes two: lo alone, mid to hi in pairs.
+// Fitted to 2000 shapes (M 256..6000, N 768..28672, K 512..14336, ranks 0 to
+// 48, group 128 and 64, all three forms, weights decoded by the call): the
+// fused kernels lie within 4-8% of it, the DMA tiles within 8-13% (5th to 95th
+// percentile).
+struct TileCost {
+  int bm, bn;
+  double lo, mid, hi, fill, rank, swiglu, call;  // mid = 0: one tile a CU
+};
+double tile_us(const TileCost& c, const GemmParams& p, int64_t P) {
+  const int64_t n = st::cdiv(p.M, c.bm) * st::cdiv(P, c.bn), cus = cu_count();
+  const double ks = (double)st::cdiv(p.Q, BK);
+  const double fill = c.fill + (p.T ? c.rank * p.lora_k : 0) + (p.swi_gu ? c.swiglu : 0);
+  if (c.mid == 0) {
+    const int64_t rest = n % cus;
+    const double occ = (double)rest / (double)cus;
+    return c.call + (double)(n / cus) * (c.hi * ks + fill) +
+           (rest ? (c.lo + (c.hi - c.lo) * occ * occ * occ) * ks + fill * (0.5 + 0.5 * occ) : 0);
+  }
+  const int64_t rest = n % (2 * cus);
+  const double us = c.call + (double)(n / (2 * cus)) * (c.hi * ks + 1.5 * fill);
+  const double occ = (double)rest / (double)cus;
+  if (rest == 0) return us;
+  if (rest <= cus) return us + c.lo * ks + fill * (0.5 + 0.5 * occ);
+  return us + (c.mid + (c.hi - c.mid) * (occ - 1)) * ks + fill * (0.5 + 0.5 * occ);
 }
 
-// Tile of a DMA GEMM: the one with the least modelled time.  Microseconds per
-// k-step and round, measured over M = 256..4096 at the four projection shapes
-// of a 4096/14336-wide layer (transposed B in brackets): a 256x256 tile 1.12
-// (1.15) on a half-idle chip rising to 1.45 (1.5) with every CU busy, where
-// the clock drops (2048 x 4096 x 4096 79 us, 4096 x 4096 x 4096 98); 256x128
-// 0.68 to 0.83 (0.72 to 0.88; 2048 x 4096 x 4096 58 us); a pair of 128x128
-// tiles on a CU 0.7 to 0.87, one alone 0.63 (512 x 4096 x 4096 47 us).
+// Tile of a DMA GEMM: the one with the least modelled time of those whose LDS
+// holds the LoRA operands (and the SwiGLU staging); 0: none does.
 // A lone 128x128 tile over a long contraction waits for memory with its two
 // slots (a vocabulary's rows: nothing of W is in a cache), so from 256 k-steps
-// it takes four: 0.5 to 0.56.  dX of a 152064-row head, hidden 4096: 64 rows
+// it takes four.  dX of a 152064-row head, hidden 4096: 64 rows
 // 1901 -> 1213 us, 256 rows 2068 -> 1348, 1024 rows 2000 -> 1319; 32000 rows,
 // 64 rows 321 -> 261.  Operands that stay in L2 gain nothing and pay for the
 // longer prologue (500 x 256 x 7168 forward 57 -> 60 us, 500 x 2048 x 128 6.5
 // -> 7.3), hence the line at 256.
 // ST_GEMM_DMA = 256, 2561, 128 or 1284 pins a tile for the tests.
-DmaKind dma_kind(bool nn, int64_t M, int64_t P, int64_t Q, double* us = nullptr) {
-  const double ks = (double)st::cdiv(Q, BK);
-  const int64_t cus = cu_count(), n128 = st::cdiv(M, 128) * st::cdiv(P, 128);
-  const double c256 = rounds_us(st::cdiv(M, 256) * st::cdiv(P, 256), cus, nn ? 1.15 : 1.12,
-                                nn ? 1.5 : 1.45, ks);
-  const double c2561 = rounds_us(st::cdiv(M, 256) * st::cdiv(P, 128), cus, nn ? 0.72 : 0.68,
-                                 nn ? 0.88 : 0.83, ks);
-  const bool deep = n128 <= cus && ks >= 256;
-  const double c128 = deep ? (nn ? 0.56 : 0.55) * ks + 5
-                      : n128 <= cus ? (nn ? 0.68 : 0.63) * ks + 5
-                                  : rounds_us(n128, 2 * cus, nn ? 0.72 : 0.7, nn ? 0.92 : 0.87, ks);
-  DmaKind k = DMA_256;
-  double c = c256;
-  if (c2561 < c) c = c2561, k = DMA_256x128;
-  if (c128 < c) c = c128, k = deep ? DMA_128_DEEP : DMA_128;
-  if (us) *us = c;
+template <bool NN>
+int dma_tile(const GemmParams& p, double* us = nullptr) {
+  struct Kind {
+    int kind, waves, lds16;
+    bool (*fits)(const GemmParams&, int64_t, int);
+    TileCost cost;
+  };
+  static const Kind kinds[] = {
+      {DMA_256, 8, st::DmaLoop256<NN, false>::LDS16, lora_staged_fits<NN, 256, 256>,
+       NN ? TileCost{256, 256, 1.07, 0, 1.34, 6.3, 0.59, 15, 11}
+          : TileCost{256, 256, 1.03, 0, 1.26, 8.7, 0.73, 0, 10}},
+      {DMA_256x128, 8, st::DmaLoop64<NN, false, 4, 2, 3>::LDS16, lora_staged_fits<NN, 256, 128>,
+       NN ? TileCost{256, 128, 0.70, 0, 0.86, 5.0, 0.29, 7, 8}
+          : TileCost{256, 128, 0.64, 0, 0.72, 6.4, 0.37, 0, 8}},
+      {DMA_128, 4, st::DmaLoop64<NN, false, 2, 2, 2>::LDS16, lora_staged_fits<NN, 128, 128>,
+       NN ? TileCost{128, 128, 0.69, 0.77, 0.95, 3.9, 0.20, 3, 7}
+          : TileCost{128, 128, 0.63, 0.66, 0.84, 4.3, 0.24, 0, 8}},
+      {DMA_128_DEEP, 4, st::DmaLoop64<NN, false, 2, 2, 4>::LDS16, lora_staged_fits<NN, 128, 128>,
+       NN ? TileCost{128, 128, 0.47, 0, 0.47, 1.7, 0.28, 3, 11}
+          : TileCost{128, 128, 0.44, 0, 0.44, 4.2, 0.32, 0, 9}}};
   const char* env = getenv("ST_GEMM_DMA");
-  const int e = env ? atoi(env) : 0;
-  return e == DMA_256 || e == DMA_256x128 || e == DMA_128 || e == DMA_128_DEEP ? (DmaKind)e : k;
+  const int pin = env ? atoi(env) : 0;
+  const bool pinned = pin == DMA_256 || pin == DMA_256x128 || pin == DMA_128 || pin == DMA_128_DEEP;
+  const bool deep = st::cdiv(p.M, 128) * st::cdiv(p.P, 128) <= cu_count() &&
+                    st::cdiv(p.Q, BK) >= 256;
+  int best = 0;
+  double least = 0;
+  for (const Kind& k : kinds) {
+    if (pinned ? k.kind != pin : k.kind == (deep ? DMA_128 : DMA_128_DEEP)) continue;
+    if (!k.fits(p, (int64_t)k.lds16 * 4, k.waves)) continue;
+    const double t = tile_us(k.cost, p, p.P);
+    if (!best || t < least) best = k.kind, least = t;
+  }
+  if (us) *us = least;
+  return best;
 }
 
 // PERM: the contraction order of the register-operand forward (gemm_dma.h)
 template <bool NN, bool PERM = false>
 int launch_dma(const GemmParams& p, hipStream_t stream) {
-  switch (dma_kind(NN, p.M, p.P, p.Q)) {
+  switch (dma_tile<NN>(p)) {
     case DMA_256: return launch_dma_tile<st::DmaLoop256<NN, PERM>>(p, stream);
     case DMA_256x128: return launch_dma_tile<st::DmaLoop64<NN, PERM, 4, 2, 3>>(p, stream);
     case DMA_128_DEEP: return launch_dma_tile<st::DmaLoop64<NN, PERM, 2, 2, 4>>(p, stream);
@@ -1983,68 +2015,60 @@ int launch_dma(const GemmParams& p, hipStream_t stream) {
   }
 }
 
-// Whether the LoRA operands (and the SwiGLU staging) fit the chosen tile.
-template <bool NN>
-bool dma_lora_fits(const GemmParams& p) {
-  switch (dma_kind(NN, p.M, p.P, p.Q)) {
-    case DMA_256:
-      return lora_staged_fits<NN, 256, 256>(p, (int64_t)st::DmaLoop256<NN, false>::LDS16 * 4, 8);
-    case DMA_256x128:
-      return lora_staged_fits<NN, 256, 128>(p, (int64_t)st::DmaLoop64<NN, false, 4, 2, 3>::LDS16 * 4, 8);
-    case DMA_128_DEEP:
-      return lora_staged_fits<NN, 128, 128>(p, (int64_t)st::DmaLoop64<NN, false, 2, 2, 4>::LDS16 * 4, 4);
-    default:
-      return lora_staged_fits<NN, 128, 128>(p, (int64_t)st::DmaLoop64<NN, false, 2, 2, 2>::LDS16 * 4, 4);
+// Modelled microseconds of the kernel that dequantises inside the GEMM, the
+// one `dispatch` would launch.  Operands beyond what the caches hold cost
+// their way to HBM on top, here and in decode_first.
+template <int MODE>
+double fused_us(const GemmParams& p) {
+  static constexpr bool NN = MODE == DGRAD_Q4;
+  static const TileCost rb{256, 256, 1.20, 0, 1.68, 10.3, 0.45, 0, 3},
+      lds256{256, 256, 1.48, 0, 2.01, 10.4, 0.47, 0, 4},
+      ws = NN ? TileCost{256, 128, 0.75, 0, 1.02, 10.8, 0.24, 7, 2}
+              : TileCost{256, 128, 0.76, 0, 0.93, 10.9, 0.37, 0, 3},
+      t128 = NN ? TileCost{128, 128, 0.79, 1.19, 1.24, 4.7, 0.25, 4, 4}
+                : TileCost{128, 128, 0.82, 1.20, 1.44, 2.8, 0.26, 0, 6},
+      flat = NN ? TileCost{128, 128, 1.04, 1.61, 1.64, 2.1, 0.21, 5, 6}
+                : TileCost{128, 128, 1.15, 1.83, 1.83, 3.8, 0.21, 0, 5};
+  const double far_bytes = (double)p.P * p.Q * 0.53 + (double)p.M * p.Q * 2 - 192e6;
+  const double far = far_bytes > 0 ? far_bytes * 0.2e-6 : 0;
+  if (p.ldw % (1 << p.gshift)) return far + tile_us(flat, p, p.P);
+  switch (tile_choice(MODE, p.M, p.P)) {
+    case 256: {
+      const TileCost& c = rb_fits(p) ? rb : lds256;
+      const int64_t c1 = split_column(256, p.M, p.P);
+      return far + (c1 ? tile_us(c, p, c1) + tile_us(ws, p, p.P - c1) : tile_us(c, p, p.P));
+    }
+    case 2562: return far + tile_us(ws, p, p.P);
+    default: return far + tile_us(t128, p, p.P);
   }
 }
 
-// Whether a dense 4-bit linear decodes W into the workspace once and runs the
-// DMA GEMM on it (the fused kernels decode every W panel once per row tile).
-// Both sides are modelled from the same measurements: the decode moves 2.53 B
-// a weight at 4.7 TB/s; the fused kernels take, per k-step and round, 1.4 to
-// 1.72 us for a 256x256 forward tile, 0.85 to 1.04 for the warp-specialised
-// 256x128 and 0.85 (dgrad 0.8) for 128x128, half as much again where scale
-// groups straddle W's rows.  At 2048 rows of a 4096/14336-wide layer with
-// rank-16 LoRA, fused against decode + GEMM: down forward 252 -> 223 us, o 85
-// -> 75, down dgrad with the SwiGLU VJP 319 -> 272, gate|up forward 478
-// against 472; at 2103 rows (a ninth row tile) down 407 -> 275, gate|up dgrad
-// 789 -> 564; at 4096 rows gate|up forward 802 -> 753, dgrad 929 -> 719.  Few
-// rows of a wide W stay fused (256 rows of gate|up 76 against 128), as do
-// fewer than 256 rows and split-K shapes (few outputs, long contraction).
+// Whether a dense 4-bit linear (p: its sizes, group, LoRA widths and form)
+// decodes W into the workspace once and runs the DMA GEMM on it (the fused
+// kernels decode every W panel once per row tile).  The decode moves 2.53 B a
+// weight at 4.7 TB/s.  At 2048 rows of a 4096/14336-wide layer with rank-16
+// LoRA, fused against decode + GEMM: down forward 252 -> 223 us, o 85 -> 75,
+// down dgrad with the SwiGLU VJP 319 -> 272; at 2103 rows (a ninth row tile)
+// down 407 -> 275, gate|up dgrad 789 -> 564; at 4096 rows gate|up forward 802
+// -> 753, dgrad 929 -> 719.  Few rows of a wide W stay fused (256 rows of
+// gate|up 76 against 128), as do fewer than 256 rows and split-K shapes (few
+// outputs, long contraction; the SwiGLU form never splits).
+// Over 1624 of the shapes that the model was fitted to, 1118 decode first: 16%
+// less time on average than always fused, and 15 of them lose more than 3% by
+// it (a model that took every weight to have 128-element groups, every row a
+// full tile and no LoRA: 14%, 119).
 // ST_GEMM_DECODE = 0 or 1 overrides the model.
 template <int MODE>
-bool decode_first(int64_t M, int64_t P, int64_t Q) {
+bool decode_first(const GemmParams& p) {
   if (getenv("ST_GEMM_TILE")) return false;
+  double dma;
+  if (!dma_tile<MODE == DGRAD_Q4>(p, &dma)) return false;
   const char* env = getenv("ST_GEMM_DECODE");
   if (env) return atoi(env) != 0;
-  if (M < 256 || split_plan(M, P, Q).splits > 1) return false;
-  constexpr bool NN = MODE == DGRAD_Q4;
-  double dma;
-  dma_kind(NN, M, P, Q, &dma);
-  dma += (double)P * (double)Q * 2.53 / 4.7e6 + 1;
-  const double ks = (double)st::cdiv(Q, BK);
-  const int64_t K = NN ? P : Q, cus = cu_count();
-  double fused;
-  if (K % 128) {
-    fused = rounds_us(st::cdiv(M, 128) * st::cdiv(P, 128), cus, 1.25, 1.25, ks);
-  } else {
-    switch (tile_choice(MODE, M, P)) {
-      case 256: {
-        const int64_t n = st::cdiv(M, 256) * st::cdiv(P, 256);
-        fused = split_column(256, M, P) ? ((double)(n / cus) + 0.6) * (1.72 * ks + 5)
-                                        : rounds_us(n, cus, 1.4, 1.72, ks);
-        break;
-      }
-      case 2562:
-        fused = rounds_us(st::cdiv(M, 256) * st::cdiv(P, 128), cus, 0.85, 1.04, ks);
-        break;
-      default: {
-        const double t = NN ? 0.8 : 0.85;
-        fused = rounds_us(st::cdiv(M, 128) * st::cdiv(P, 128), cus, t, t, ks);
-      }
-    }
-  }
-  return dma < fused;
+  if (p.M < 256 || (!p.swi_gu && split_plan(p.M, p.P, p.Q).splits > 1)) return false;
+  const double far_bytes = 2.0 * ((double)p.P + (double)p.M) * (double)p.Q - 192e6;
+  dma += (double)p.P * (double)p.Q * 0.54e-6 + (far_bytes > 0 ? far_bytes * 0.4e-6 : 0);
+  return dma * 1.01 < fused_us<MODE>(p);
 }
 int64_t decode_workspace(int64_t N, int64_t K) { return N * K * 2 + 256; }
 
@@ -2068,16 +2092,35 @@ int decode_and_run(GemmParams p, const uint8_t* payload, const float* scales, in
 }  // namespace
 
 // Every shape also runs from the packed weight without a workspace.
+extern "C" int64_t st_q4_linear_workspace_bytes(int32_t form, int64_t M, int64_t N, int64_t K,
+                                                int32_t flags, int32_t rank, int64_t lora_cols,
+                                                int64_t max_decode_bytes) {
+  if (M <= 0 || N <= 0 || K <= 0 || form < ST_Q4_FWD || form > ST_Q4_DGRAD_SWIGLU) return 0;
+  const bool fwd = form == ST_Q4_FWD;
+  // sizes only: the pointers say which operands there are
+  GemmParams p{};
+  p.M = M; p.P = fwd ? N : K; p.Q = fwd ? K : N;
+  p.ldw = K;
+  p.gshift = (flags & ST_FLAG_GROUP64) ? 6 : 7;
+  if (rank > 0) {
+    p.T = p.L = (const float*)sizeof(float);
+    p.lora_k = rank;
+    p.lora_cols = (int)std::min<int64_t>(lora_cols, 1 << 20);
+  }
+  if (form == ST_Q4_DGRAD_SWIGLU) p.swi_gu = (const uint16_t*)sizeof(float);
+  const int64_t decode = decode_workspace(N, K);
+  if ((max_decode_bytes < 0 || decode <= max_decode_bytes) &&
+      (fwd ? decode_first<FWD_Q4>(p) : decode_first<DGRAD_Q4>(p)))
+    return decode;
+  return p.swi_gu ? 0 : split_workspace(split_plan(M, p.P, p.Q), M, p.P);
+}
+
 extern "C" int64_t st_q4_linear_fwd_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (decode_first<FWD_Q4>(M, N, K)) return decode_workspace(N, K);
-  return split_workspace(split_plan(M, N, K), M, N);
+  return st_q4_linear_workspace_bytes(ST_Q4_FWD, M, N, K, 0, 0, 0, -1);
 }
 
 extern "C" int64_t st_q4_linear_dgrad_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (decode_first<DGRAD_Q4>(M, K, N)) return decode_workspace(N, K);
-  return split_workspace(split_plan(M, K, N), M, K);
+  return st_q4_linear_workspace_bytes(ST_Q4_DGRAD, M, N, K, 0, 0, 0, -1);
 }
 
 static int check_lora_common(int64_t rank, int64_t cols) {
@@ -2133,8 +2176,7 @@ extern "C" int st_q4_linear_fwd(const uint16_t* x, int64_t M, int64_t K, int64_t
   ST_CHECK_ARG(((uintptr_t)payload & 3u) == 0, "st_q4_linear_fwd: payload not 4-byte aligned");
   p.Wq = payload; p.Ws = scales; p.ldw = K;
   p.w_bytes = N * K / 2; p.s_bytes = st::cdiv(N * K, 1ll << p.gshift) * 4;
-  if (workspace && decode_first<FWD_Q4>(M, N, K) && workspace_bytes >= decode_workspace(N, K) &&
-      dma_lora_fits<false>(p))
+  if (workspace && workspace_bytes >= decode_workspace(N, K) && decode_first<FWD_Q4>(p))
     return decode_and_run<false>(p, payload, scales, N, lut16, flags, workspace, s);
   if (K % (1 << p.gshift) == 0 && al16(payload)) {
     // split-K when the caller brought the workspace the query asks for
@@ -2187,8 +2229,7 @@ static int dgrad_impl(const uint16_t* dy, int64_t M, int64_t N, int64_t lddy,
   ST_CHECK_ARG(((uintptr_t)payload & 3u) == 0, "st_q4_linear_dgrad: payload not 4-byte aligned");
   p.Wq = payload; p.Ws = scales; p.ldw = K;
   p.w_bytes = N * K / 2; p.s_bytes = st::cdiv(N * K, 1ll << p.gshift) * 4;
-  if (workspace && decode_first<DGRAD_Q4>(M, K, N) && workspace_bytes >= decode_workspace(N, K) &&
-      dma_lora_fits<true>(p))
+  if (workspace && workspace_bytes >= decode_workspace(N, K) && decode_first<DGRAD_Q4>(p))
     return decode_and_run<true>(p, payload, scales, N, lut16, flags, workspace, s);
   if (K % (1 << p.gshift) == 0) {
     // split-K (not with the SwiGLU VJP) when the caller brought the workspace

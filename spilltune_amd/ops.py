@@ -207,15 +207,17 @@ class _Workspace:
 _ws = _Workspace()
 
 
-def _gemm_scratch(device, nbytes: int) -> torch.Tensor | None:
+def _gemm_scratch(weight: Q4Weight, form: int, M: int, rank: int, cols: int):
     """Scratch of one fused GEMM call (decoded weights or split-K partials),
     from the caching allocator, so that it belongs to the current stream.  None
     when nothing is needed or the device has no room for it: the call then
     decodes inside the GEMM."""
+    N, K = weight.shape
+    nbytes = _lib.query("st_q4_linear_workspace_bytes", form, M, N, K, weight.flags, rank, cols, -1)
     if nbytes <= 0:
         return None
     try:
-        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+        return torch.empty(nbytes, dtype=torch.uint8, device=weight.device)
     except torch.OutOfMemoryError:
         return None
 
@@ -388,7 +390,7 @@ class _Q4LoRALinear(torch.autograd.Function):
             ends = _lib.i64_array(list(accumulate(weight.segments)))
         # W decoded once for many rows, or split-K partials for shapes whose
         # tiles leave CUs idle (0 otherwise)
-        ws = _gemm_scratch(dev, _lib.query("st_q4_linear_fwd_workspace_bytes", M, N, K))
+        ws = _gemm_scratch(weight, _lib.ST_Q4_FWD, M, rank if ab else 0, nseg * rank)
         _launch(("fwd", M, N, K), lambda: _lib.call(
             "st_q4_linear_fwd", _lib.ptr(x), M, K, K, _lib.ptr(weight.payload),
             _lib.ptr(weight.scales), N, weight.lut(), weight.flags,
@@ -499,10 +501,11 @@ class _Q4LoRALinear(torch.autograd.Function):
             _clear_missing(dT, ctx.loras, rank)
         lora_args = (_lib.ptr(dT), 0 if dT is None else dT.stride(0), _lib.ptr(A_cat),
                      0 if dT is None else dT.shape[1])
+        ws = _gemm_scratch(weight, _lib.ST_Q4_DGRAD_SWIGLU if ctx.swiglu_I else _lib.ST_Q4_DGRAD, M,
+                           lora_args[3], lora_args[3])
         if ctx.swiglu_I:
             # the dgrad epilogue applies the SwiGLU VJP: the gradient of gate|up
             dx = torch.empty_like(gu)
-            ws = _gemm_scratch(dev, _lib.query("st_q4_linear_dgrad_workspace_bytes", M, N, K))
             _launch(("dgrad", M, N, K), lambda: _lib.call(
                 "st_q4_linear_dgrad_swiglu", _lib.ptr(dy), M, N, N, _lib.ptr(weight.payload),
                 _lib.ptr(weight.scales), K, weight.lut(), weight.flags, *lora_args,
@@ -510,7 +513,6 @@ class _Q4LoRALinear(torch.autograd.Function):
                 0 if ws is None else ws.numel(), stream))
         else:
             dx = torch.empty((M, K), dtype=_BF16, device=dev)
-            ws = _gemm_scratch(dev, _lib.query("st_q4_linear_dgrad_workspace_bytes", M, N, K))
             _launch(("dgrad", M, N, K), lambda: _lib.call(
                 "st_q4_linear_dgrad", _lib.ptr(dy), M, N, N, _lib.ptr(weight.payload),
                 _lib.ptr(weight.scales), K, weight.lut(), weight.flags, *lora_args,

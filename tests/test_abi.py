@@ -55,6 +55,27 @@ def test_lut_array_keeps_the_sign_of_zero():
     assert bytes(_lib.lut_array(range(16))) == bytes((ctypes.c_float * 16)(*range(16)))
 
 
+def test_linear_workspace_query_knows_the_call():
+    """The workspace that is asked for is one the call would use."""
+    def q(form, M, N, K, flags=0, rank=0, cols=0, limit=-1):
+        return _lib.query("st_q4_linear_workspace_bytes", form, M, N, K, flags, rank, cols, limit)
+    fwd, dgrad, swiglu = _lib.ST_Q4_FWD, _lib.ST_Q4_DGRAD, _lib.ST_Q4_DGRAD_SWIGLU
+    g64 = _lib.ST_FLAG_GROUP64
+    down = (4096, 14336)  # [N, K]
+    assert q(fwd, 2048, *down) == q(fwd, 2048, *down, rank=16, cols=16) == 2 * 4096 * 14336 + 256
+    # the SwiGLU form never splits the contraction: no partials, decode or nothing
+    assert 0 < q(dgrad, 256, *down) != 2 * 4096 * 14336 + 256
+    assert q(swiglu, 256, *down) in (0, 2 * 4096 * 14336 + 256)
+    # 64-element groups do not straddle rows of 1088, 128-element groups do
+    assert q(fwd, 300, 8000, 1088, flags=g64) == 0 < q(fwd, 1000, 8000, 1088)
+    # more LoRA columns than any tile holds beside the DMA rings
+    assert q(fwd, 2048, *down, rank=128, cols=128) == 0
+    assert q(dgrad, 2048, *down, rank=192, cols=192) == 0
+    assert q(fwd, 2048, *down, limit=2 * 4096 * 14336 + 255) == 0
+    assert q(fwd, 2048, *down, limit=2 * 4096 * 14336 + 256) > 0
+    assert q(3, 2048, *down) == q(-1, 2048, *down) == q(fwd, 0, *down) == 0
+
+
 def test_lora_rank_limits_rejected_before_any_launch():
     """Rank bounds of the LoRA entry points: checked on the host, before any
     device work (fake pointers never reach a kernel)."""

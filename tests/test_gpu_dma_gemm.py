@@ -118,24 +118,33 @@ def test_decode_first_linear_gives_the_fused_bits(dev, monkeypatch, tile, M, N, 
     A = torch.randn(nseg * rank, K, device=dev, generator=g) if rank else None
     ends = _lib.i64_array([N * (i + 1) // nseg for i in range(nseg)])
 
+    W, ws = w.dequantize(), torch.empty(2 * N * K + 256, dtype=torch.uint8, device=dev)
+    start = -ws.data_ptr() % 256
+
+    def call(decode, name, form, *args):
+        wa = (P(ws), ws.numel()) if decode else (None, 0)
+        ws.fill_(0xA5)
+        _lib.call(name, *args, *wa, st)
+        # the workspace then holds W's decode, on every tile that the query says
+        # it runs on: all but the 64 KiB one with 64 LoRA columns
+        need = _lib.query("st_q4_linear_workspace_bytes", form, M, N, K, flags, rank,
+                          rank * nseg, -1)
+        decodes = decode and not (tile == "128" and rank * nseg == 64)
+        assert torch.equal(ws[start:start + 2 * N * K].view(BF).view(N, K), W) == decodes, name
+        assert not decode or need == (ws.numel() if decodes else 0), name
+
     def run(decode):
         monkeypatch.setenv("ST_GEMM_DECODE", str(int(decode)))
-        ws = None
-        if decode:
-            need = _lib.query("st_q4_linear_fwd_workspace_bytes", M, N, K)
-            assert need >= 2 * N * K
-            ws = torch.empty(need, dtype=torch.uint8, device=dev)
-        wa = (P(ws), 0 if ws is None else ws.numel(), st)
         y, dx, dgu = torch.empty_like(dy), torch.empty_like(x), torch.empty_like(gu)
         lf = (P(T), nseg * rank, P(B), rank, 0.5, nseg, ends) if rank else (None, 0, None, 0, 1.0,
                                                                             0, None)
         lb = (P(T), nseg * rank, P(A), nseg * rank) if rank else (None, 0, None, 0)
-        _lib.call("st_q4_linear_fwd", P(x), M, K, K, P(w.payload), P(w.scales), N, w.lut(), flags,
-                  *lf, P(res), N, P(y), N, *wa)
-        _lib.call("st_q4_linear_dgrad", P(dy), M, N, N, P(w.payload), P(w.scales), K, w.lut(),
-                  flags, *lb, P(dx), K, *wa)
-        _lib.call("st_q4_linear_dgrad_swiglu", P(dy), M, N, N, P(w.payload), P(w.scales), K,
-                  w.lut(), flags, *lb, P(gu), 2 * K, P(dgu), 2 * K, *wa)
+        call(decode, "st_q4_linear_fwd", _lib.ST_Q4_FWD, P(x), M, K, K, P(w.payload),
+             P(w.scales), N, w.lut(), flags, *lf, P(res), N, P(y), N)
+        call(decode, "st_q4_linear_dgrad", _lib.ST_Q4_DGRAD, P(dy), M, N, N, P(w.payload),
+             P(w.scales), K, w.lut(), flags, *lb, P(dx), K)
+        call(decode, "st_q4_linear_dgrad_swiglu", _lib.ST_Q4_DGRAD_SWIGLU, P(dy), M, N, N,
+             P(w.payload), P(w.scales), K, w.lut(), flags, *lb, P(gu), 2 * K, P(dgu), 2 * K)
         return y, dx, dgu
 
     fused = run(False)
