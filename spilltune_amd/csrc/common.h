@@ -136,43 +136,32 @@ __device__ __forceinline__ bf16x8 tr_operand(const uint4* bs, int n0, int kc, in
 
 // XCD-aware block remap: consecutive logical tiles land on the same XCD so they
 // share that XCD's L2 (blocks are dispatched round-robin over the 8 XCDs).
-__device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t nb) {
+__device__ __forceinline__ unsigned xcd_remap(unsigned b, unsigned nb) {
   if (nb % 8 != 0) return b;
   return (b % 8) * (nb / 8) + b / 8;
 }
 
 // Tile (row tile mt, column tile pt) of logical tile t in a grouped raster:
 // logical tiles walk `gm` row tiles for each column tile before the next
-// column tile, group after group of gm row tiles (gm <= 1: row-major, the
+// column tile, group after group of gm row tiles (gm = 1: row-major, the
 // column tile fastest).  With xcd_remap, an XCD's consecutive logical tiles
 // then cover gm row panels x (its share / gm) column panels, so its L2 serves
-// each A panel and each W panel to several of its CUs.
-__device__ __forceinline__ void raster(int64_t t, int64_t tiles_m, int64_t tiles_p, int gm,
+// each A panel and each W panel to several of its CUs.  In 32 bits (a launch
+// has less than 2^31 tiles): 64-bit divisions cost about 1 us a workgroup.
+// Grouped (per-expert) launches, whose row-tile slots past the last expert's
+// exit at once, take gm = 8 on a multiple of 8 slots and no remap: slot mt
+// goes to XCD mt % 8 (its column tiles one after the other there, sharing the
+// expert's A rows in that L2), so the empty slots at the end fall on all XCDs
+// alike.  Contiguous runs of slots per XCD left the last XCDs with nothing but
+// empty ones (256 experts of ~64 rows: 384 slots of 128 rows, 96 of them on
+// two XCDs without work).
+constexpr unsigned GROUPED_RASTER = 8;
+__device__ __forceinline__ void raster(unsigned t, unsigned tiles_m, unsigned tiles_p, unsigned gm,
                                        int64_t& mt, int64_t& pt) {
-  if (gm <= 1) {
-    mt = t / tiles_p;
-    pt = t % tiles_p;
-    return;
-  }
-  const int64_t per = (int64_t)gm * tiles_p;
-  const int64_t m0 = t / per * gm, r = t % per;
-  const int64_t h = tiles_m - m0 < gm ? tiles_m - m0 : gm;  // rows of a short last group
+  const unsigned per = gm * tiles_p, m0 = t / per * gm, r = t % per;
+  const unsigned h = min(tiles_m - m0, gm);  // rows of a short last group
   mt = m0 + r % h;
   pt = r / h;
-}
-
-// Tile of workgroup b of a grouped launch, whose row-tile slots past the last
-// group's exit at once: slot mt goes to XCD mt % 8 (its column tiles one after
-// the other there, sharing the group's A rows in that L2), so the empty slots
-// at the end fall on all XCDs alike.  Contiguous runs of slots per XCD left
-// the last XCDs with nothing but empty ones (256 experts of ~64 rows: 384
-// slots of 128 rows, 96 of them on two XCDs without work).  The grid holds a
-// multiple of 8 slots.
-__device__ __forceinline__ void grouped_raster(unsigned b, unsigned tiles_p, int64_t& mt,
-                                               int64_t& pt) {
-  const unsigned i = b / 8;
-  mt = (int64_t)(i / tiles_p) * 8 + b % 8;
-  pt = i % tiles_p;
 }
 
 // Grouped (per-expert) row tiles: group g owns rows [off[g], off[g+1]) and

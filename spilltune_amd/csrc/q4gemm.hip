@@ -73,8 +73,8 @@ struct GemmParams {
   // and moves 16-byte rows (C, residual, gate|up 16-byte aligned with row
   // strides and P multiples of 8, and the staging fits the tile's LDS)
   int vec_epi;
-  // row tiles per raster group (st::raster); grouped launches take 1
-  int raster_m;
+  // set by the launcher: row tiles per raster group (st::raster), and in all
+  unsigned raster_m, tiles_m;
   // split-K (gemm_ws_kernel, dense launches): the grid holds `splits` copies
   // of the tiles, copy s taking contraction k-steps [s*ks_len, (s+1)*ks_len),
   // and each writes its raw fp32 sums to part[s][M][P] (no epilogue);
@@ -710,11 +710,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_kernel(GemmParams p) {
   const int wm = wave / TL::WAVES_N, wn = wave % TL::WAVES_N;
   const int64_t tiles_p = st::cdiv(p.P, BN);
   int64_t mt, pt;
-  if (p.goff)
-    st::grouped_raster(blockIdx.x, (unsigned)tiles_p, mt, pt);
-  else
-    st::raster(st::xcd_remap(blockIdx.x, gridDim.x), st::cdiv(p.M, BM), tiles_p, p.raster_m, mt,
-               pt);
+  st::raster(p.goff ? blockIdx.x : st::xcd_remap(blockIdx.x, gridDim.x), p.tiles_m,
+             (unsigned)tiles_p, p.raster_m, mt, pt);
   const int64_t p0 = pt * BN;
   int64_t m0 = mt * BM, mend = p.M;
   int grp = 0;
@@ -1017,24 +1014,21 @@ __global__ __launch_bounds__(512) void gemm_ws_kernel(GemmParams p) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t tiles_p = st::cdiv(p.P, BN);
-  int64_t t = st::xcd_remap(blockIdx.x, gridDim.x);
+  unsigned t = p.goff ? blockIdx.x : st::xcd_remap(blockIdx.x, gridDim.x);
   // split-K: split s covers contraction [q0, q0 + qlen) (q0 a multiple of
   // 4*BK, so ring slots and scale groups keep their phase); the operands'
   // bases move by q0 and every index below stays relative to it
   int64_t q0 = 0, qlen = p.Q;
   int split = 0;
   if (p.splits > 1) {
-    const int64_t nt = st::cdiv(p.M, BM) * tiles_p;
+    const unsigned nt = p.tiles_m * (unsigned)tiles_p;
     split = (int)(t / nt);
     t -= split * nt;
     q0 = (int64_t)split * p.ks_len * BK;
     qlen = p.Q - q0 < (int64_t)p.ks_len * BK ? p.Q - q0 : (int64_t)p.ks_len * BK;
   }
   int64_t mt, pt;
-  if (p.goff)
-    st::grouped_raster(blockIdx.x, (unsigned)tiles_p, mt, pt);
-  else
-    st::raster(t, st::cdiv(p.M, BM), tiles_p, p.raster_m, mt, pt);
+  st::raster(t, p.tiles_m, (unsigned)tiles_p, p.raster_m, mt, pt);
   const int64_t p0 = pt * BN;
   int64_t m0 = mt * BM, mend = p.M;
   int grp = 0;
@@ -1536,11 +1530,8 @@ __global__ __launch_bounds__(64 * WAVES, FM == 4 ? 4 : 1) void gemm_rb_kernel(Ge
   __shared__ uint4 ldsA[RB_ST * BM * BK / 8];
   const int64_t tiles_p = st::cdiv(p.P, BN);
   int64_t mt, pt;
-  if (p.goff)
-    st::grouped_raster(blockIdx.x, (unsigned)tiles_p, mt, pt);
-  else
-    st::raster(st::xcd_remap(blockIdx.x, gridDim.x), st::cdiv(p.M, BM), tiles_p, p.raster_m, mt,
-               pt);
+  st::raster(p.goff ? blockIdx.x : st::xcd_remap(blockIdx.x, gridDim.x), p.tiles_m,
+             (unsigned)tiles_p, p.raster_m, mt, pt);
   int64_t m0 = mt * BM, mend = p.M;
   int grp = 0;
   if (p.goff) {  // grouped (per-expert) rows: the whole workgroup leaves together
@@ -1572,14 +1563,10 @@ __global__ __launch_bounds__(LP::NT, LP::MIN_WG_WAVES) void gemm_dma_kernel(Gemm
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int M = (int)p.M, P = (int)p.P;
-  // st::xcd_remap and st::raster in 32 bits (64-bit divisions cost ~1 us here)
-  const unsigned nb = gridDim.x, tiles_m = (M + LP::BM - 1) / LP::BM,
-                 tiles_p = (P + LP::BN - 1) / LP::BN;
-  unsigned t = blockIdx.x;
-  if (nb % 8 == 0) t = (t % 8) * (nb / 8) + t / 8;
-  const unsigned per = (unsigned)p.raster_m * tiles_p, r0 = t / per * p.raster_m, r = t % per;
-  const unsigned h = min(tiles_m - r0, (unsigned)p.raster_m);
-  const int m0 = (int)(r0 + r % h) * LP::BM, p0 = (int)(r / h) * LP::BN;
+  int64_t mt, pt;
+  st::raster(st::xcd_remap(blockIdx.x, gridDim.x), p.tiles_m, (P + LP::BN - 1) / LP::BN,
+             p.raster_m, mt, pt);
+  const int m0 = (int)mt * LP::BM, p0 = (int)pt * LP::BN;
   const st::DmaOperands o{p.A, p.Wb, p.lda, p.ldw, p.a_bytes, p.w_bytes};
   f32x4 acc[LP::FM][LP::FN];
   LP::run(o, lds, m0, M, p0, P, (int)p.Q, wave, lane, acc);
@@ -1612,26 +1599,25 @@ int choose_epilogue(GemmParams& p, int64_t lds_dwords, int waves) {
   return ST_OK;
 }
 
+// Row-tile slots of a launch: grouped launches (per-expert row ranges) take
+// sum_g cdiv(rows_g, BM) <= cdiv(rows, BM) + groups, a multiple of
+// GROUPED_RASTER; slots past the last group's tiles exit at once.
+int64_t row_tiles(const GemmParams& p, int BM) {
+  const int64_t n = st::cdiv(p.M, BM);
+  return p.goff ? st::cdiv(n + p.ngroups, st::GROUPED_RASTER) * st::GROUPED_RASTER : n;
+}
+
 // Row tiles per raster group (st::raster) of a dense launch: 4, so each XCD's
 // 32 CUs take 4 row panels x 8 column panels at a time and its L2 serves each
 // A and W panel to several CUs (with row-major order one A panel and 32 W
 // panels: every XCD streamed all of W).  Measured on the Llama-8B layer step:
 // 3.84-3.86 ms with 1, 3.76 ms with 2 or 4, 3.78 ms with 8; every fused GEMM
-// of the step 1-3% faster.  ST_GEMM_RASTER overrides it; grouped launches
-// keep their expert order.
-int raster_choice(const GemmParams& p) {
-  if (p.goff) return 1;
+// of the step 1-3% faster.  ST_GEMM_RASTER overrides it (up to 64).
+void choose_raster(GemmParams& p, int BM) {
   const char* env = getenv("ST_GEMM_RASTER");
   const int g = env ? atoi(env) : 4;
-  return g > 1 ? g : 1;
-}
-
-// Row-tile slots of a launch: grouped launches (per-expert row ranges) take
-// sum_g cdiv(rows_g, BM) <= cdiv(rows, BM) + groups, a multiple of 8 for
-// st::grouped_raster; slots past the last group's tiles exit at once.
-int64_t row_tiles(const GemmParams& p, int BM) {
-  const int64_t n = st::cdiv(p.M, BM);
-  return p.goff ? st::cdiv(n + p.ngroups, 8) * 8 : n;
+  p.raster_m = p.goff ? st::GROUPED_RASTER : g > 1 ? std::min(g, 64) : 1;
+  p.tiles_m = (unsigned)row_tiles(p, BM);
 }
 
 // The epilogue addresses C, the residual, T and the LoRA right operand with
@@ -1661,7 +1647,7 @@ int launch_ws(const GemmParams& p, hipStream_t stream) {
   if (!lora_staged_fits<MODE == DGRAD_Q4, BM, BN>(p, (int64_t)WS_DA * BM * BK / 8 * 4, 4))
     return launch<MODE, 128, 128, 4>(p, stream);
   GemmParams q = p;
-  q.raster_m = raster_choice(q);
+  choose_raster(q, BM);
   if (int rc = choose_epilogue<MODE == DGRAD_Q4, BM, BN>(q, (int64_t)WS_DA * BM * BK / 8 * 4, 4))
     return rc;
   gemm_ws_kernel<MODE><<<(unsigned)tiles, 512, 0, stream>>>(q);
@@ -1681,7 +1667,7 @@ int launch_rb(const GemmParams& p, hipStream_t stream) {
   if (!lora_staged_fits<false, BM, BN>(p, lds_dwords, NT / 64))
     return launch<FWD_Q4, 128, 128, 4>(p, stream);
   GemmParams q = p;
-  q.raster_m = raster_choice(q);
+  choose_raster(q, BM);
   if (int rc = choose_epilogue<false, BM, BN>(q, lds_dwords, NT / 64)) return rc;
   if (q.hi_first)
     gemm_rb_kernel<FN, WAVES, true, FM><<<(unsigned)tiles, NT, 0, stream>>>(q);
@@ -1698,7 +1684,7 @@ int launch(const GemmParams& p, hipStream_t stream) {
   if (int rc = check_epilogue_extents(p)) return rc;
   using TL = Tile<MODE, BM, BN, WAVES, WAVES_M>;
   GemmParams q = p;
-  q.raster_m = raster_choice(q);
+  choose_raster(q, BM);
   // the LoRA epilogue stages T and the right operand in the tile's LDS when
   // they fit; otherwise the 128x128 kernel built to read them from global
   // memory runs the GEMM
@@ -1858,7 +1844,7 @@ int launch_ws_split(GemmParams p, const SplitPlan& plan, void* workspace, hipStr
   p.part = (float*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
   p.splits = plan.splits;
   p.ks_len = plan.ks_len;
-  p.raster_m = raster_choice(p);
+  choose_raster(p, 256);
   const int64_t tiles = st::cdiv(p.M, 256) * st::cdiv(p.P, 128) * plan.splits;
   if (tiles > 0x7fffffff) return st::fail(ST_EUNSUPPORTED, "q4gemm: too many tiles");
   gemm_ws_kernel<MODE><<<(unsigned)tiles, 512, 0, stream>>>(p);
@@ -1921,7 +1907,7 @@ int launch_dma_tile(GemmParams p, hipStream_t stream) {
   const int64_t tiles = st::cdiv(p.M, LP::BM) * st::cdiv(p.P, LP::BN);
   if (tiles > 0x7fffffff) return st::fail(ST_EUNSUPPORTED, "q4gemm: too many tiles");
   if (int rc = check_epilogue_extents(p)) return rc;
-  p.raster_m = raster_choice(p);
+  choose_raster(p, LP::BM);
   if (int rc = choose_epilogue<LP::NN_B, LP::BM, LP::BN>(p, (int64_t)LP::LDS16 * 4, LP::WAVES)) return rc;
   gemm_dma_kernel<LP><<<(unsigned)tiles, LP::NT, 0, stream>>>(p);
   return st::check_launch("gemm_dma");
