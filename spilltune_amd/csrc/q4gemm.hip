@@ -1913,21 +1913,22 @@ int launch_dma_tile(GemmParams p, hipStream_t stream) {
   return st::check_launch("gemm_dma");
 }
 
-// Modelled microseconds of a GEMM of `n` tiles: the cost of a 64-deep k-step
-// of a round, from a nearly idle chip (lo) to a full one (hi, where the clock
+// Modelled microseconds of a GEMM: the cost of a 64-deep k-step of a round of
+// tiles, from a nearly idle chip (lo) to a full one (hi, where the clock
 // drops), and a tile's fill (with its epilogue: per LoRA rank, and with the
 // SwiGLU VJP).  Tiles of which a CU takes two: lo alone, mid to hi in pairs.
-// Fitted to 2000 shapes (M 256..6000, N 768..28672, K 512..14336, ranks 0 to
-// 48, group 128 and 64, all three forms, weights decoded by the call): the
-// fused kernels lie within 4-8% of it, the DMA tiles within 8-13% (5th to 95th
-// percentile).
+// A contraction that is not a multiple of 64 starts A's rows off the 128-byte
+// lines: a share `ragged` more per k-step.  Fitted to 2000 shapes (M
+// 256..6000, N 768..28672, K 512..14336, ranks 0 to 48, group 128 and 64, all
+// three forms, weights decoded by the call): the fused kernels lie within 4-8%
+// of it, the DMA tiles within 6-16% (5th to 95th percentile).
 struct TileCost {
   int bm, bn;
-  double lo, mid, hi, fill, rank, swiglu, call;  // mid = 0: one tile a CU
+  double lo, mid, hi, fill, rank, swiglu, call, ragged;  // mid = 0: one tile a CU
 };
 double tile_us(const TileCost& c, const GemmParams& p, int64_t P) {
   const int64_t n = st::cdiv(p.M, c.bm) * st::cdiv(P, c.bn), cus = cu_count();
-  const double ks = (double)st::cdiv(p.Q, BK);
+  const double ks = (double)st::cdiv(p.Q, BK) * (p.Q % 64 ? 1 + c.ragged : 1);
   const double fill = c.fill + (p.T ? c.rank * p.lora_k : 0) + (p.swi_gu ? c.swiglu : 0);
   if (c.mid == 0) {
     const int64_t rest = n % cus;
@@ -1962,17 +1963,17 @@ int dma_tile(const GemmParams& p, double* us = nullptr) {
   };
   static const Kind kinds[] = {
       {DMA_256, 8, st::DmaLoop256<NN, false>::LDS16, lora_staged_fits<NN, 256, 256>,
-       NN ? TileCost{256, 256, 1.07, 0, 1.34, 6.3, 0.59, 15, 11}
-          : TileCost{256, 256, 1.03, 0, 1.26, 8.7, 0.73, 0, 10}},
+       NN ? TileCost{256, 256, 1.07, 0, 1.39, 4.6, 0.59, 15, 12, 0}
+          : TileCost{256, 256, 1.03, 0, 1.31, 7.5, 0.74, 0, 11, 0.05}},
       {DMA_256x128, 8, st::DmaLoop64<NN, false, 4, 2, 3>::LDS16, lora_staged_fits<NN, 256, 128>,
-       NN ? TileCost{256, 128, 0.70, 0, 0.86, 5.0, 0.29, 7, 8}
-          : TileCost{256, 128, 0.64, 0, 0.72, 6.4, 0.37, 0, 8}},
+       NN ? TileCost{256, 128, 0.65, 0, 0.81, 4.2, 0.29, 7, 9, 0.08}
+          : TileCost{256, 128, 0.62, 0, 0.75, 5.4, 0.37, 0, 9, 0.21}},
       {DMA_128, 4, st::DmaLoop64<NN, false, 2, 2, 2>::LDS16, lora_staged_fits<NN, 128, 128>,
-       NN ? TileCost{128, 128, 0.69, 0.77, 0.95, 3.9, 0.20, 3, 7}
-          : TileCost{128, 128, 0.63, 0.66, 0.84, 4.3, 0.24, 0, 8}},
+       NN ? TileCost{128, 128, 0.62, 0.69, 0.87, 3.2, 0.20, 3, 8, 0.12}
+          : TileCost{128, 128, 0.62, 0.65, 0.87, 3.5, 0.24, 0, 9, 0.27}},
       {DMA_128_DEEP, 4, st::DmaLoop64<NN, false, 2, 2, 4>::LDS16, lora_staged_fits<NN, 128, 128>,
-       NN ? TileCost{128, 128, 0.47, 0, 0.47, 1.7, 0.28, 3, 11}
-          : TileCost{128, 128, 0.44, 0, 0.44, 4.2, 0.32, 0, 9}}};
+       NN ? TileCost{128, 128, 0.47, 0, 0.47, 1.1, 0.28, 3, 12, 0.02}
+          : TileCost{128, 128, 0.43, 0, 0.43, 3.1, 0.32, 0, 10, 0.22}}};
   const char* env = getenv("ST_GEMM_DMA");
   const int pin = env ? atoi(env) : 0;
   const bool pinned = pin == DMA_256 || pin == DMA_256x128 || pin == DMA_128 || pin == DMA_128_DEEP;
@@ -2001,22 +2002,28 @@ int launch_dma(const GemmParams& p, hipStream_t stream) {
   }
 }
 
+// Operand bytes beyond what the caches hold, which rows off the 128-byte lines
+// fetch again (4846 x 19640 x 4480 dgrad decoded first, 256x128 tiles: 1096 us,
+// with 19648 columns 856).
+double far_bytes(const GemmParams& p, double w_bytes) {
+  const double far = w_bytes + 2.0 * (double)p.M * (double)p.Q - 192e6;
+  return p.Q % 64 && far > 0 ? far : 0;
+}
+
 // Modelled microseconds of the kernel that dequantises inside the GEMM, the
-// one `dispatch` would launch.  Operands beyond what the caches hold cost
-// their way to HBM on top, here and in decode_first.
+// one `dispatch` would launch.
 template <int MODE>
 double fused_us(const GemmParams& p) {
   static constexpr bool NN = MODE == DGRAD_Q4;
-  static const TileCost rb{256, 256, 1.20, 0, 1.68, 10.3, 0.45, 0, 3},
-      lds256{256, 256, 1.48, 0, 2.01, 10.4, 0.47, 0, 4},
-      ws = NN ? TileCost{256, 128, 0.75, 0, 1.02, 10.8, 0.24, 7, 2}
-              : TileCost{256, 128, 0.76, 0, 0.93, 10.9, 0.37, 0, 3},
-      t128 = NN ? TileCost{128, 128, 0.79, 1.19, 1.24, 4.7, 0.25, 4, 4}
-                : TileCost{128, 128, 0.82, 1.20, 1.44, 2.8, 0.26, 0, 6},
-      flat = NN ? TileCost{128, 128, 1.04, 1.61, 1.64, 2.1, 0.21, 5, 6}
-                : TileCost{128, 128, 1.15, 1.83, 1.83, 3.8, 0.21, 0, 5};
-  const double far_bytes = (double)p.P * p.Q * 0.53 + (double)p.M * p.Q * 2 - 192e6;
-  const double far = far_bytes > 0 ? far_bytes * 0.2e-6 : 0;
+  static const TileCost rb{256, 256, 1.18, 0, 1.69, 10.3, 0.46, 0, 3, 0.05},
+      lds256{256, 256, 1.48, 0, 2.00, 10.6, 0.47, 0, 4, 0.05},
+      ws = NN ? TileCost{256, 128, 0.75, 0, 1.01, 10.6, 0.24, 7, 2, 0.02}
+              : TileCost{256, 128, 0.77, 0, 0.93, 11.4, 0.37, 0, 2, 0.05},
+      t128 = NN ? TileCost{128, 128, 0.78, 1.18, 1.25, 4.1, 0.25, 4, 5, 0}
+                : TileCost{128, 128, 0.82, 1.20, 1.44, 2.5, 0.25, 0, 7, 0.05},
+      flat = NN ? TileCost{128, 128, 1.02, 1.60, 1.60, 2.2, 0.21, 5, 6, 0.02}
+                : TileCost{128, 128, 1.12, 1.76, 1.76, 3.3, 0.21, 0, 6, 0.04};
+  const double far = 0.2e-6 * far_bytes(p, (double)p.P * p.Q * 0.53);
   if (p.ldw % (1 << p.gshift)) return far + tile_us(flat, p, p.P);
   switch (tile_choice(MODE, p.M, p.P)) {
     case 256: {
@@ -2039,10 +2046,10 @@ double fused_us(const GemmParams& p) {
 // -> 753, dgrad 929 -> 719.  Few rows of a wide W stay fused (256 rows of
 // gate|up 76 against 128), as do fewer than 256 rows and split-K shapes (few
 // outputs, long contraction; the SwiGLU form never splits).
-// Over 1624 of the shapes that the model was fitted to, 1118 decode first: 16%
-// less time on average than always fused, and 15 of them lose more than 3% by
-// it (a model that took every weight to have 128-element groups, every row a
-// full tile and no LoRA: 14%, 119).
+// Over the 2030 shapes that the model was fitted to, 1470 decode first: 16%
+// less time on average than always fused, and 34 of them lose more than 3% by
+// it (a model that took every weight to have 128-element groups and the
+// register-operand kernel, without fills, ragged rows and LoRA: 13%, a tenth).
 // ST_GEMM_DECODE = 0 or 1 overrides the model.
 template <int MODE>
 bool decode_first(const GemmParams& p) {
@@ -2052,9 +2059,9 @@ bool decode_first(const GemmParams& p) {
   const char* env = getenv("ST_GEMM_DECODE");
   if (env) return atoi(env) != 0;
   if (p.M < 256 || (!p.swi_gu && split_plan(p.M, p.P, p.Q).splits > 1)) return false;
-  const double far_bytes = 2.0 * ((double)p.P + (double)p.M) * (double)p.Q - 192e6;
-  dma += (double)p.P * (double)p.Q * 0.54e-6 + (far_bytes > 0 ? far_bytes * 0.4e-6 : 0);
-  return dma * 1.01 < fused_us<MODE>(p);
+  const double w = (double)p.P * (double)p.Q;
+  dma += w * 0.54e-6 + 0.4e-6 * far_bytes(p, 2 * w);
+  return dma < fused_us<MODE>(p);
 }
 int64_t decode_workspace(int64_t N, int64_t K) { return N * K * 2 + 256; }
 
