@@ -160,12 +160,18 @@ def ptr(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 
 
-def stream_handle(device: torch.device | None = None) -> int:
+def stream_handle(device: torch.device | str | int | None = None) -> int:
     """The current stream's handle (an int, as every pointer argument takes)
-    without building a Stream object: a layer step asks for it ~40 times."""
-    if device is not None and device.type != "cuda":
-        raise ValueError(f"Expected a cuda device, but got: {device}")
-    index = device.index if device is not None else None
+    without building a Stream object: a layer step asks for it ~40 times.
+    ``device`` as for torch.cuda.current_stream."""
+    if isinstance(device, str):
+        device = torch.device(device)
+    if isinstance(device, torch.device):
+        if device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        index = device.index
+    else:
+        index = device
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None
                                               else index)
 

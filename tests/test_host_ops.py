@@ -5,7 +5,7 @@ scanned on the host)."""
 import pytest
 import torch
 
-from spilltune_amd import ops
+from spilltune_amd import _lib, ops
 
 
 def _q4(payload, scales, rows, K=128):
@@ -84,3 +84,15 @@ def test_router_parts_sum_exactly_and_follow_the_version():
     assert again is not parts
     back = again[:E].double() + again[E:2 * E].double() + again[2 * E:].double()
     assert torch.equal(back, w.double())
+
+
+def test_stream_handle_takes_what_current_stream_takes(monkeypatch):
+    """A torch.device, its name, an index or nothing; only CUDA devices."""
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 1000 + i, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 7)
+    h = _lib.stream_handle
+    assert h() == h(None) == h("cuda") == h(torch.device("cuda")) == 1007
+    assert h(2) == h("cuda:2") == h(torch.device("cuda", 2)) == 1002
+    for bad in ("cpu", torch.device("cpu")):
+        with pytest.raises(ValueError, match="cuda device"):
+            h(bad)
