@@ -39,13 +39,18 @@ _F32 = torch.float32
 @dataclass
 class Q4Weight:
     """A frozen ``[out, in]`` 4-bit matrix resident on the device (views into a
-    slot).  ``segments`` lists the out-widths of N-concatenated projections."""
+    slot).  ``segments`` lists the out-widths of N-concatenated projections.
+    ``decode_limit`` bounds the scratch in bytes (``2 * out * in + 256``) that a
+    GEMM with many rows may decode it into; 0 keeps every decode inside the
+    GEMM, None sets no bound.  The result is the same either way, but for the
+    last bit of the fp32 LoRA term."""
     payload: torch.Tensor
     scales: torch.Tensor
     shape: tuple
     codec: str
     segments: tuple = field(default=())
     flags: int = 0
+    decode_limit: int | None = None
 
     def __post_init__(self):
         self.shape = tuple(int(s) for s in self.shape)
@@ -141,8 +146,10 @@ def concat_rows(weights) -> Q4Weight | None:
         base_p.untyped_storage(), base_p.storage_offset(), (rows * K // 2,), (1,))
     scales = torch.empty(0, dtype=_F32, device=base_s.device).set_(
         base_s.untyped_storage(), base_s.storage_offset(), (rows * K // first.group,), (1,))
+    limits = [w.decode_limit for w in weights if w.decode_limit is not None]
     return Q4Weight(payload, scales, (rows, K), first.codec,
-                    tuple(w.out_features for w in weights), first.flags)
+                    tuple(w.out_features for w in weights), first.flags,
+                    min(limits) if limits else None)
 
 
 # ----------------------------------------------------------------- timing hook
@@ -208,17 +215,25 @@ _ws = _Workspace()
 
 
 def _gemm_scratch(weight: Q4Weight, form: int, M: int, rank: int, cols: int):
-    """Scratch of one fused GEMM call (decoded weights or split-K partials),
-    from the caching allocator, so that it belongs to the current stream.  None
-    when nothing is needed or the device has no room for it: the call then
-    decodes inside the GEMM."""
+    """Scratch of one fused GEMM call (decoded weights within the weight's
+    ``decode_limit``, or split-K partials), from the caching allocator, so that
+    it belongs to the current stream; None when the call needs none.  Without
+    room on the device for the decoded weights the call decodes inside the
+    GEMM; split-K partials, without which the fp32 sums would run in another
+    order, are not given up."""
     N, K = weight.shape
-    nbytes = _lib.query("st_q4_linear_workspace_bytes", form, M, N, K, weight.flags, rank, cols, -1)
+
+    def need(limit):
+        return _lib.query("st_q4_linear_workspace_bytes", form, M, N, K, weight.flags, rank, cols,
+                          limit)
+    nbytes = need(-1 if weight.decode_limit is None else max(0, weight.decode_limit))
     if nbytes <= 0:
         return None
     try:
         return torch.empty(nbytes, dtype=torch.uint8, device=weight.device)
     except torch.OutOfMemoryError:
+        if need(0) > 0:
+            raise
         return None
 
 

@@ -126,7 +126,7 @@ def pack_image(block: BlockPlan, layout: SlotLayout, out: torch.Tensor) -> None:
             out[o:o + nb].copy_(block.host_weights[name].contiguous().view(torch.uint8).reshape(-1))
 
 
-def views_of(buffer: torch.Tensor, layout: SlotLayout) -> dict:
+def views_of(buffer: torch.Tensor, layout: SlotLayout, decode_limit: int | None = None) -> dict:
     """Weight views over a device (or host) image: Q4Weight for 4-bit
     matrices, Q4Experts for packed 3-D expert stacks [E, N, K]."""
     from .moe import Q4Experts
@@ -138,7 +138,7 @@ def views_of(buffer: torch.Tensor, layout: SlotLayout) -> dict:
             if len(shape) == 3:
                 views[name] = Q4Experts(payload, scales, shape[0], shape[1], shape[2], codec)
             else:
-                views[name] = Q4Weight(payload, scales, shape, codec)
+                views[name] = Q4Weight(payload, scales, shape, codec, decode_limit=decode_limit)
         else:
             _, dtype, shape, o, nb = e
             views[name] = buffer[o:o + nb].view(dtype).view(shape)
@@ -157,7 +157,10 @@ class _Lease:
 
 
 class Q4SlotSession:
-    """Two (or more) device slots of packed layer images with one-layer lookahead."""
+    """Two (or more) device slots of packed layer images with one-layer lookahead.
+    ``device_budget_bytes`` bounds the slots and, with what they leave of it,
+    the scratch that a GEMM with many rows decodes one of their weights into
+    (``Q4Weight.decode_limit``); activations and adapters are not counted."""
 
     asynchronous = True
 
@@ -176,6 +179,7 @@ class Q4SlotSession:
             raise MemoryError("resource_budget: pinned block images exceed the host limit")
         if self.capacity * slots > device_budget_bytes:
             raise MemoryError("resource_budget: device slots exceed the device limit")
+        self.decode_limit = device_budget_bytes - self.capacity * slots
         if slots < 1 or (len(self.blocks) > 1 and slots < 2):
             raise MemoryError("resource_budget: a multi-block plan needs two slots")
         self.positions = {id(b): i for i, b in enumerate(self.blocks)}
@@ -281,7 +285,7 @@ class Q4SlotSession:
             slot["buffer"][:layout.nbytes].copy_(img, non_blocking=True)
             ready.record(self.copy_stream)
         slot["ready"] = ready
-        slot["views"] = views_of(slot["buffer"], layout)
+        slot["views"] = views_of(slot["buffer"], layout, self.decode_limit)
         record.update(start_event=start, ready_event=ready)
         self.copy_records.append(record)
         self.transferred_bytes += layout.nbytes

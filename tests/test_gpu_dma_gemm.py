@@ -179,3 +179,37 @@ def test_decode_first_rule_and_small_workspace(dev):
                   _lib.ptr(y), N, _lib.ptr(ws), nbytes, _lib.stream_handle(dev))
         ys.append(y)
     assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
+
+
+def test_slot_budget_bounds_the_decoded_weights(dev):
+    """A session whose slots take its whole device budget decodes inside the
+    GEMMs: the same bits, no scratch of a decoded matrix on the device."""
+    from spilltune_amd import codecs, slots
+    N, K, M = 4096, 2048, 2103
+    host_w = torch.randn(N, K, generator=torch.Generator().manual_seed(1)) * 0.02
+    rec = codecs.encode(host_w.to(BF), "nf4-g128")
+    name = "self_attn.o_proj.weight"
+    host = {f"@{name}/{part}": t for part, t in rec.parts.items()}
+    specs = {name: {"spec": rec.spec, "parts": {part: f"@{name}/{part}" for part in rec.parts}}}
+    block = slots.BlockPlan(0, "full_attention", None, {}, host, {}, specs)
+    g = torch.Generator(device=dev).manual_seed(2)
+    x = _rand(g, M, K)
+    probe = slots.Q4SlotSession([block], dev, host_budget_bytes=1 << 30,
+                                device_budget_bytes=1 << 30)
+    got = []
+    for budget in (2 * probe.capacity, 1 << 30):
+        session = slots.Q4SlotSession([block], dev, host_budget_bytes=1 << 30,
+                                      device_budget_bytes=budget)
+        with session.run():
+            with session.reloader(block).borrow("forward") as views:
+                w = views[name]
+                assert w.decode_limit == budget - 2 * probe.capacity
+                torch.cuda.synchronize()
+                torch.cuda.reset_peak_memory_stats(dev)
+                before = torch.cuda.memory_allocated(dev)
+                y = ops.q4_lora_linear(x, w, None)
+                torch.cuda.synchronize()
+                got.append((y, torch.cuda.max_memory_allocated(dev) - before))
+    (y0, peak0), (y1, peak1) = got
+    assert torch.equal(y0, y1)
+    assert peak0 < 2 * M * N + (1 << 20) and peak1 - peak0 >= 2 * N * K  # y, and the decoded W

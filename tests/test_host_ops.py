@@ -96,3 +96,39 @@ def test_stream_handle_takes_what_current_stream_takes(monkeypatch):
     for bad in ("cpu", torch.device("cpu")):
         with pytest.raises(ValueError, match="cuda device"):
             h(bad)
+
+
+def test_gemm_scratch_is_bounded(monkeypatch):
+    """Decoded weights stay within the weight's limit (the tighter one of a
+    concatenation), and give way when the device has no room; split-K partials
+    do not (without them the sums run in another order)."""
+    empty = torch.empty(0, dtype=torch.uint8)
+    N, K = 4096, 14336
+    decode = 2 * N * K + 256
+
+    def scratch(form, M, limit=None):
+        ws = ops._gemm_scratch(ops.Q4Weight(empty, empty, (N, K), "nf4-g128", decode_limit=limit),
+                               form, M, 0, 0)
+        return 0 if ws is None else ws.numel()
+    split = scratch(_lib.ST_Q4_DGRAD, 256)
+    assert scratch(_lib.ST_Q4_FWD, 2048) == decode != split > 0
+    assert scratch(_lib.ST_Q4_FWD, 2048, decode) == decode
+    assert scratch(_lib.ST_Q4_FWD, 2048, decode - 1) == scratch(_lib.ST_Q4_FWD, 2048, 0) == 0
+    assert scratch(_lib.ST_Q4_FWD, 2048, -5) == 0
+    assert scratch(_lib.ST_Q4_DGRAD, 256, 0) == split
+
+    payload, scales = torch.zeros(128 * 64, dtype=torch.uint8), torch.zeros(128)
+    a, b = (_q4(payload[i * 4096:], scales[i * 64:], 64) for i in (0, 1))
+    a.payload, a.scales = payload[:4096], scales[:64]
+    assert ops.concat_rows([a, b]).decode_limit is None
+    a.decode_limit, b.decode_limit = None, 7
+    assert ops.concat_rows([a, b]).decode_limit == 7
+    a.decode_limit = 3
+    assert ops.concat_rows([a, b]).decode_limit == 3
+
+    def full(*args, **kwargs):
+        raise torch.OutOfMemoryError("full")
+    monkeypatch.setattr(torch, "empty", full)
+    assert scratch(_lib.ST_Q4_FWD, 2048) == 0
+    with pytest.raises(torch.OutOfMemoryError):
+        scratch(_lib.ST_Q4_DGRAD, 256)
