@@ -194,24 +194,12 @@ def _launch(key, fn):
 
 
 # ----------------------------------------------------------------- workspace
-class _Workspace:
-    """Per-device scratch grown on demand through the PyTorch allocator."""
-
-    def __init__(self):
-        self._buf = {}
-
-    def get(self, device, nbytes: int) -> torch.Tensor | None:
-        if nbytes <= 0:
-            return None
-        key = (device.type, device.index)
-        buf = self._buf.get(key)
-        if buf is None or buf.numel() < nbytes:
-            buf = torch.empty(int(nbytes * 1.25) + 256, dtype=torch.uint8, device=device)
-            self._buf[key] = buf
-        return buf
-
-
-_ws = _Workspace()
+def _scratch(device, nbytes: int) -> torch.Tensor | None:
+    """Scratch of one call from the caching allocator: it belongs to the current
+    stream and to nobody else, so calls on other streams or threads, and graphs
+    that captured an earlier one, never share it (one torch.empty is ~2 us of
+    host time)."""
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes > 0 else None
 
 
 def _gemm_scratch(weight: Q4Weight, form: int, M: int, rank: int, cols: int):
@@ -240,7 +228,7 @@ def _gemm_scratch(weight: Q4Weight, form: int, M: int, rank: int, cols: int):
 def lora_gemm(Mo, No, Kc, a, sam, sak, b, sbk, sbn, alpha, out, accumulate=False):
     """``out = (accumulate ? out : 0) + alpha * sum_k a(m,k) b(k,n)`` (fp32 out)."""
     need = _lib.query("st_lora_gemm_workspace_bytes", Mo, No, Kc)
-    ws = _ws.get(out.device, need)
+    ws = _scratch(out.device, need)
     dt = {_BF16: _lib.ST_DTYPE_BF16, _F32: _lib.ST_DTYPE_F32}
     _lib.call("st_lora_gemm", Mo, No, Kc, _lib.ptr(a), dt[a.dtype], sam, sak, _lib.ptr(b),
               dt[b.dtype], sbk, sbn, float(alpha), _lib.ptr(out), out.stride(0), int(accumulate),
@@ -292,7 +280,8 @@ class LoraGradSink:
             chunk = self.products[i:i + 16]
             arr = (_lib.RkProduct * len(chunk))(*chunk)
             need = _lib.query("st_rk_batch_workspace_bytes", len(chunk), arr)
-            ws = _ws.get(self.device, need)
+            with torch.cuda.stream(self.stream):
+                ws = _scratch(self.device, need)
             _lib.call("st_rk_batch", len(chunk), arr, _lib.ptr(ws),
                       0 if ws is None else ws.numel(), st)
         # the operands may be freed before the products finish: the allocator
@@ -455,7 +444,7 @@ class _Q4LoRALinear(torch.autograd.Function):
             ends = _lib.i64_array(starts[1:])
             need = _lib.query("st_lora_bwd_dy_workspace_bytes", M, N, rank, nseg, ends)
             if need > 0:
-                ws = _ws.get(dev, need)
+                ws = _scratch(dev, need)
                 _lib.call("st_lora_bwd_dy", _lib.ptr(dy), M, N, N, _lib.ptr(B_cat), _lib.ptr(T),
                           T.stride(0), rank, nseg, ends, float(scale), _lib.ptr(dT), dT.stride(0),
                           None, _lib.ptr(ws), ws.numel(), stream)
@@ -486,7 +475,7 @@ class _Q4LoRALinear(torch.autograd.Function):
             ends = _lib.i64_array(list(accumulate(weight.segments)))
             need = _lib.query("st_lora_bwd_dy_workspace_bytes", M, N, rank, nseg, ends)
             if need > 0:
-                ws = _ws.get(dev, need)
+                ws = _scratch(dev, need)
                 _lib.call("st_lora_bwd_dy", _lib.ptr(dy), M, N, N, _lib.ptr(B_cat), _lib.ptr(T),
                           T.stride(0), rank, nseg, ends, float(scale), _lib.ptr(dT), dT.stride(0),
                           _lib.ptr(dB_all), _lib.ptr(ws), ws.numel(), stream)
@@ -896,7 +885,7 @@ class _CausalAttention(torch.autograd.Function):
         dev = q.device
         out = torch.empty((B, S, H * D), dtype=_BF16, device=dev)
         lse = torch.empty((B, H, S), dtype=_F32, device=dev)
-        ws = _ws.get(dev, _lib.query("st_flash_attn_workspace_bytes", B, S, H, Hkv, D, 0))
+        ws = _scratch(dev, _lib.query("st_flash_attn_workspace_bytes", B, S, H, Hkv, D, 0))
         _lib.call("st_flash_attn_fwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), B, S, H, Hkv, D,
                   float(scale), _lib.ptr(kv_len), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(ws),
                   0 if ws is None else ws.numel(), _lib.stream_handle(dev))
@@ -912,7 +901,7 @@ class _CausalAttention(torch.autograd.Function):
         dev = q.device
         dout = dout.contiguous()
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        ws = _ws.get(dev, _lib.query("st_flash_attn_workspace_bytes", B, S, H, Hkv, D, 1))
+        ws = _scratch(dev, _lib.query("st_flash_attn_workspace_bytes", B, S, H, Hkv, D, 1))
         _lib.call("st_flash_attn_bwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out),
                   _lib.ptr(lse), _lib.ptr(dout), B, S, H, Hkv, D, float(ctx.scale),
                   _lib.ptr(ctx.kv_len), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(ws),
@@ -995,7 +984,7 @@ class _MLAAttention(torch.autograd.Function):
         dev = q.device
         out = torch.empty((B, S, H * DV), dtype=_BF16, device=dev)
         lse = torch.empty((B, H, S), dtype=_F32, device=dev)
-        ws = _ws.get(dev, _lib.query("st_mla_attn_workspace_bytes", B, S, H, DQ, DV, 0))
+        ws = _scratch(dev, _lib.query("st_mla_attn_workspace_bytes", B, S, H, DQ, DV, 0))
         _lib.call("st_mla_attn_fwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), B, S, H, DQ, DV,
                   float(scale), _lib.ptr(kv_len), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(ws),
                   0 if ws is None else ws.numel(), _lib.stream_handle(dev))
@@ -1011,7 +1000,7 @@ class _MLAAttention(torch.autograd.Function):
         dev = q.device
         dout = dout.contiguous()
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        ws = _ws.get(dev, _lib.query("st_mla_attn_workspace_bytes", B, S, H, DQ, DV, 1))
+        ws = _scratch(dev, _lib.query("st_mla_attn_workspace_bytes", B, S, H, DQ, DV, 1))
         _lib.call("st_mla_attn_bwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out),
                   _lib.ptr(lse), _lib.ptr(dout), B, S, H, DQ, DV, float(ctx.scale),
                   _lib.ptr(ctx.kv_len), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(ws),

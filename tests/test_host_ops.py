@@ -2,6 +2,8 @@
 (CPU only): when fused projections may share one weight view, and the
 terminal's label rules (native_terminal.py:39-47: device labels are never
 scanned on the host)."""
+import threading
+
 import pytest
 import torch
 
@@ -132,3 +134,27 @@ def test_gemm_scratch_is_bounded(monkeypatch):
     assert scratch(_lib.ST_Q4_FWD, 2048) == 0
     with pytest.raises(torch.OutOfMemoryError):
         scratch(_lib.ST_Q4_DGRAD, 256)
+
+
+def test_calls_in_flight_do_not_share_scratch(monkeypatch):
+    """Two calls that overlap (two threads or two streams) get workspaces of
+    their own: the second must not write its partials over the first's."""
+    barrier, seen = threading.Barrier(2, timeout=30), []
+
+    def call(name, *args):
+        seen.append((args[-3], args[-2]))  # workspace and its size; the stream is last
+        barrier.wait()  # both calls have their workspace in hand
+    monkeypatch.setattr(_lib, "call", call)
+    monkeypatch.setattr(_lib, "stream_handle", lambda device=None: 0)
+    x, A, T = torch.zeros(64, 2048), torch.zeros(8, 2048), torch.zeros(64, 8)
+    assert _lib.query("st_lora_gemm_workspace_bytes", 64, 8, 2048) > 0
+    for _ in range(2):  # also with a buffer that an earlier call left behind
+        threads = [threading.Thread(target=ops.lora_gemm,
+                                    args=(64, 8, 2048, x, 2048, 1, A, 1, 2048, 1.0, T))
+                   for _ in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    for (a, size), (b, _) in (seen[:2], seen[2:]):
+        assert abs(a - b) >= size > 0
