@@ -110,6 +110,7 @@ EXPORTED = tuple(_SIGNATURES)
 
 _lock = threading.Lock()
 _lib = None
+_fns: dict = {}  # the library's bound functions, once it is loaded
 
 
 class KernelError(RuntimeError):
@@ -118,7 +119,7 @@ class KernelError(RuntimeError):
 
 def load():
     """Load and bind the library once; raise loudly when it is absent."""
-    global _lib
+    global _lib, _fns
     if _lib is not None:
         return _lib
     with _lock:
@@ -134,7 +135,7 @@ def load():
                 fn.argtypes = args
             if lib.st_abi_version() != 1:
                 raise RuntimeError("dependency: libspilltune_hip.so ABI version mismatch")
-            _lib = lib
+            _lib, _fns = lib, {name: getattr(lib, name) for name in _SIGNATURES}
     return _lib
 
 
@@ -147,13 +148,19 @@ def check(rc: int, what: str) -> None:
     raise KernelError(f"{what}: {msg}")
 
 
+def _bound() -> dict:
+    load()
+    return _fns
+
+
 def call(name: str, *args) -> None:
-    lib = load()
-    check(getattr(lib, name)(*args), name)
+    rc = (_fns or _bound())[name](*args)
+    if rc != ST_OK:
+        check(rc, name)
 
 
 def query(name: str, *args) -> int:
-    return int(getattr(load(), name)(*args))
+    return (_fns or _bound())[name](*args)
 
 
 def ptr(t: torch.Tensor | None):

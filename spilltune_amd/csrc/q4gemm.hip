@@ -1802,35 +1802,41 @@ SplitPlan split_plan(int64_t M, int64_t P, int64_t Q) {
   SplitPlan plan;
   const char* env = getenv("ST_GEMM_SPLITK");
   if (env && atoi(env) == 0) return plan;
-  const int64_t tiles = st::cdiv(M, 256) * st::cdiv(P, 128), KT = st::cdiv(Q, BK);
-  const int64_t cus = cu_count();
+  const int64_t tiles64 = st::cdiv(M, 256) * st::cdiv(P, 128), cus = cu_count();
+  const unsigned KT = (unsigned)st::cdiv(Q, BK), tiles = (unsigned)std::min(tiles64, cus);
   if (KT < 16 || P % 4 || M * P * 4 >= (1ll << 31)) return plan;
   if (!env && (getenv("ST_GEMM_TILE") || 2.0 * (double)M * (double)P * (double)Q < 8e9))
     return plan;
-  auto shape = [&](int64_t s, int64_t& len) {
-    len = st::cdiv(st::cdiv(KT, s), 4) * 4;
-    return st::cdiv(KT, len);
+  auto cdiv = [](unsigned a, unsigned b) { return (a + b - 1) / b; };
+  auto shape = [&](unsigned s, unsigned& len) {
+    len = cdiv(cdiv(KT, s), 4) * 4;
+    return cdiv(KT, len);
   };
-  auto cost = [&](int64_t s) {
-    int64_t len;
-    const int64_t ns = shape(s, len);
-    return st::cdiv(tiles * ns, cus) * (len + 8);
+  auto cost = [&](unsigned s) {
+    unsigned len;
+    const unsigned ns = shape(s, len);
+    return cdiv(tiles * ns, (unsigned)cus) * (len + 8);
   };
-  int64_t best = 1, bc = cost(1);
+  unsigned best = 1, bc = cost(1);
   if (env) {
-    best = atoi(env);
+    best = (unsigned)std::max(1, atoi(env));
   } else {
-    if (tiles >= cus) return plan;
-    for (int64_t s = 2; s <= 32; ++s)
+    if (tiles64 >= cus) return plan;
+    for (unsigned s = 2; s <= 32; ++s)
       if (cost(s) < bc) bc = cost(s), best = s;
     if (best == 1 || bc * 4 > cost(1) * 3) return plan;
   }
-  int64_t len;
-  const int64_t ns = shape(best, len);
+  unsigned len;
+  const unsigned ns = shape(best, len);
   if (ns <= 1) return plan;
   plan.splits = (int)ns;
   plan.ks_len = (int)len;
   return plan;
+}
+
+// the plan of a dense 4-bit linear: the SwiGLU form never splits
+SplitPlan linear_split(const GemmParams& p) {
+  return p.swi_gu ? SplitPlan{} : split_plan(p.M, p.P, p.Q);
 }
 
 int64_t split_workspace(const SplitPlan& plan, int64_t M, int64_t P) {
@@ -1926,8 +1932,8 @@ struct TileCost {
   int bm, bn;
   double lo, mid, hi, fill, rank, swiglu, call, ragged;  // mid = 0: one tile a CU
 };
-double tile_us(const TileCost& c, const GemmParams& p, int64_t P) {
-  const int64_t n = st::cdiv(p.M, c.bm) * st::cdiv(P, c.bn), cus = cu_count();
+double tile_us(const TileCost& c, const GemmParams& p, int64_t P, int64_t cus) {
+  const int64_t n = st::cdiv(p.M, c.bm) * st::cdiv(P, c.bn);
   const double ks = (double)st::cdiv(p.Q, BK) * (p.Q % 64 ? 1 + c.ragged : 1);
   const double fill = c.fill + (p.T ? c.rank * p.lora_k : 0) + (p.swi_gu ? c.swiglu : 0);
   if (c.mid == 0) {
@@ -1977,14 +1983,14 @@ int dma_tile(const GemmParams& p, double* us = nullptr) {
   const char* env = getenv("ST_GEMM_DMA");
   const int pin = env ? atoi(env) : 0;
   const bool pinned = pin == DMA_256 || pin == DMA_256x128 || pin == DMA_128 || pin == DMA_128_DEEP;
-  const bool deep = st::cdiv(p.M, 128) * st::cdiv(p.P, 128) <= cu_count() &&
-                    st::cdiv(p.Q, BK) >= 256;
+  const int64_t cus = cu_count();
+  const bool deep = st::cdiv(p.M, 128) * st::cdiv(p.P, 128) <= cus && st::cdiv(p.Q, BK) >= 256;
   int best = 0;
   double least = 0;
   for (const Kind& k : kinds) {
     if (pinned ? k.kind != pin : k.kind == (deep ? DMA_128 : DMA_128_DEEP)) continue;
     if (!k.fits(p, (int64_t)k.lds16 * 4, k.waves)) continue;
-    const double t = tile_us(k.cost, p, p.P);
+    const double t = tile_us(k.cost, p, p.P, cus);
     if (!best || t < least) best = k.kind, least = t;
   }
   if (us) *us = least;
@@ -2024,15 +2030,17 @@ double fused_us(const GemmParams& p) {
       flat = NN ? TileCost{128, 128, 1.02, 1.60, 1.60, 2.2, 0.21, 5, 6, 0.02}
                 : TileCost{128, 128, 1.12, 1.76, 1.76, 3.3, 0.21, 0, 6, 0.04};
   const double far = 0.2e-6 * far_bytes(p, (double)p.P * p.Q * 0.53);
-  if (p.ldw % (1 << p.gshift)) return far + tile_us(flat, p, p.P);
+  const int64_t cus = cu_count();
+  if (p.ldw % (1 << p.gshift)) return far + tile_us(flat, p, p.P, cus);
   switch (tile_choice(MODE, p.M, p.P)) {
     case 256: {
       const TileCost& c = rb_fits(p) ? rb : lds256;
       const int64_t c1 = split_column(256, p.M, p.P);
-      return far + (c1 ? tile_us(c, p, c1) + tile_us(ws, p, p.P - c1) : tile_us(c, p, p.P));
+      return far + (c1 ? tile_us(c, p, c1, cus) + tile_us(ws, p, p.P - c1, cus)
+                       : tile_us(c, p, p.P, cus));
     }
-    case 2562: return far + tile_us(ws, p, p.P);
-    default: return far + tile_us(t128, p, p.P);
+    case 2562: return far + tile_us(ws, p, p.P, cus);
+    default: return far + tile_us(t128, p, p.P, cus);
   }
 }
 
@@ -2052,13 +2060,13 @@ double fused_us(const GemmParams& p) {
 // register-operand kernel, without fills, ragged rows and LoRA: 13%, a tenth).
 // ST_GEMM_DECODE = 0 or 1 overrides the model.
 template <int MODE>
-bool decode_first(const GemmParams& p) {
+bool decode_first(const GemmParams& p, const SplitPlan& plan) {
   if (getenv("ST_GEMM_TILE")) return false;
+  const char* env = getenv("ST_GEMM_DECODE");
+  if (env ? !atoi(env) : p.M < 256 || plan.splits > 1) return false;
   double dma;
   if (!dma_tile<MODE == DGRAD_Q4>(p, &dma)) return false;
-  const char* env = getenv("ST_GEMM_DECODE");
-  if (env) return atoi(env) != 0;
-  if (p.M < 256 || (!p.swi_gu && split_plan(p.M, p.P, p.Q).splits > 1)) return false;
+  if (env) return true;
   const double w = (double)p.P * (double)p.Q;
   dma += w * 0.54e-6 + 0.4e-6 * far_bytes(p, 2 * w);
   return dma < fused_us<MODE>(p);
@@ -2101,11 +2109,12 @@ extern "C" int64_t st_q4_linear_workspace_bytes(int32_t form, int64_t M, int64_t
     p.lora_cols = (int)std::min<int64_t>(lora_cols, 1 << 20);
   }
   if (form == ST_Q4_DGRAD_SWIGLU) p.swi_gu = (const uint16_t*)sizeof(float);
+  const SplitPlan plan = linear_split(p);
   const int64_t decode = decode_workspace(N, K);
   if ((max_decode_bytes < 0 || decode <= max_decode_bytes) &&
-      (fwd ? decode_first<FWD_Q4>(p) : decode_first<DGRAD_Q4>(p)))
+      (fwd ? decode_first<FWD_Q4>(p, plan) : decode_first<DGRAD_Q4>(p, plan)))
     return decode;
-  return p.swi_gu ? 0 : split_workspace(split_plan(M, p.P, p.Q), M, p.P);
+  return split_workspace(plan, M, p.P);
 }
 
 extern "C" int64_t st_q4_linear_fwd_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -2169,12 +2178,12 @@ extern "C" int st_q4_linear_fwd(const uint16_t* x, int64_t M, int64_t K, int64_t
   ST_CHECK_ARG(((uintptr_t)payload & 3u) == 0, "st_q4_linear_fwd: payload not 4-byte aligned");
   p.Wq = payload; p.Ws = scales; p.ldw = K;
   p.w_bytes = N * K / 2; p.s_bytes = st::cdiv(N * K, 1ll << p.gshift) * 4;
-  if (workspace && workspace_bytes >= decode_workspace(N, K) && decode_first<FWD_Q4>(p))
+  const SplitPlan plan = workspace ? linear_split(p) : SplitPlan{};
+  if (workspace && workspace_bytes >= decode_workspace(N, K) && decode_first<FWD_Q4>(p, plan))
     return decode_and_run<false>(p, payload, scales, N, lut16, flags, workspace, s);
   if (K % (1 << p.gshift) == 0 && al16(payload)) {
     // split-K when the caller brought the workspace the query asks for
-    const SplitPlan plan = split_plan(M, N, K);
-    if (plan.splits > 1 && workspace && workspace_bytes >= split_workspace(plan, M, N))
+    if (plan.splits > 1 && workspace_bytes >= split_workspace(plan, M, N))
       return launch_ws_split<FWD_Q4>(p, plan, workspace, s);
     return dispatch<FWD_Q4>(p, s);
   }
@@ -2222,12 +2231,12 @@ static int dgrad_impl(const uint16_t* dy, int64_t M, int64_t N, int64_t lddy,
   ST_CHECK_ARG(((uintptr_t)payload & 3u) == 0, "st_q4_linear_dgrad: payload not 4-byte aligned");
   p.Wq = payload; p.Ws = scales; p.ldw = K;
   p.w_bytes = N * K / 2; p.s_bytes = st::cdiv(N * K, 1ll << p.gshift) * 4;
-  if (workspace && workspace_bytes >= decode_workspace(N, K) && decode_first<DGRAD_Q4>(p))
+  const SplitPlan plan = workspace ? linear_split(p) : SplitPlan{};
+  if (workspace && workspace_bytes >= decode_workspace(N, K) && decode_first<DGRAD_Q4>(p, plan))
     return decode_and_run<true>(p, payload, scales, N, lut16, flags, workspace, s);
   if (K % (1 << p.gshift) == 0) {
     // split-K (not with the SwiGLU VJP) when the caller brought the workspace
-    const SplitPlan plan = split_plan(M, K, N);
-    if (!gu && plan.splits > 1 && workspace && workspace_bytes >= split_workspace(plan, M, K))
+    if (plan.splits > 1 && workspace_bytes >= split_workspace(plan, M, K))
       return launch_ws_split<DGRAD_Q4>(p, plan, workspace, s);
     return dispatch<DGRAD_Q4>(p, s);
   }

@@ -24,6 +24,7 @@ import math
 from contextlib import contextmanager
 
 from dataclasses import dataclass, field
+from functools import lru_cache
 from itertools import accumulate
 
 import torch
@@ -36,6 +37,12 @@ _F32 = torch.float32
 
 
 # ----------------------------------------------------------------- weights
+@lru_cache(maxsize=None)
+def _codec_lut(codec: str):
+    """A codec's codebook for the C ABI (read only; the codecs are few)."""
+    return _lib.lut_array(codebook(codec))
+
+
 @dataclass
 class Q4Weight:
     """A frozen ``[out, in]`` 4-bit matrix resident on the device (views into a
@@ -81,7 +88,7 @@ class Q4Weight:
         return 64 if self.flags & _lib.ST_FLAG_GROUP64 else GROUP
 
     def lut(self):
-        return _lib.lut_array(codebook(self.codec))
+        return _codec_lut(self.codec)
 
     def dequantize(self) -> torch.Tensor:
         """bf16 copy of the matrix (for checks / reference-side use only)."""
@@ -210,17 +217,15 @@ def _gemm_scratch(weight: Q4Weight, form: int, M: int, rank: int, cols: int):
     GEMM; split-K partials, without which the fp32 sums would run in another
     order, are not given up."""
     N, K = weight.shape
-
-    def need(limit):
-        return _lib.query("st_q4_linear_workspace_bytes", form, M, N, K, weight.flags, rank, cols,
-                          limit)
-    nbytes = need(-1 if weight.decode_limit is None else max(0, weight.decode_limit))
+    limit = -1 if weight.decode_limit is None else max(0, weight.decode_limit)
+    nbytes = _lib.query("st_q4_linear_workspace_bytes", form, M, N, K, weight.flags, rank, cols,
+                        limit)
     if nbytes <= 0:
         return None
     try:
         return torch.empty(nbytes, dtype=torch.uint8, device=weight.device)
     except torch.OutOfMemoryError:
-        if need(0) > 0:
+        if _lib.query("st_q4_linear_workspace_bytes", form, M, N, K, weight.flags, rank, cols, 0) > 0:
             raise
         return None
 
