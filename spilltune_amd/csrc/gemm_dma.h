@@ -5,8 +5,9 @@
 //
 // What bounds it: at full load the card lowers its clock (a 4096^3 product
 // takes 106 us on random operands and 78 us on zeros, the same instructions),
-// so bytes moved per flop count as much as latency.  The 256x256 tile reads
-// 24 KiB of LDS per 2 MFLOP and wave against 32 KiB for the 256x128 tile;
+// so bytes moved per flop count as much as latency.  A 128x64 wave tile (256x256)
+// reads 24 KiB of LDS per k-step of 1 MFLOP, the 64x64 one (256x128) 16 KiB
+// per half of that;
 // 16x16x32 ran 4-5% faster than 32x32x16 at full load (down-projection shape
 // 2048 x 4096 x 14336: 186 against 194 us), and equally fast on zeros.
 #pragma once
